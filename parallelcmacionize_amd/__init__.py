@@ -572,9 +572,9 @@ class WarmStartNet:
         self._check(self.lib.cmi_net_set_input_mode(self.h, int(mode)))
 
     def set_tiled(self, on):
-        """Forward convolutions through the LDS-tiled kernel where the
-        volume divides into its blocks (default), or always through the
-        per-run kernel; the outputs are identical."""
+        """Forward convolutions through the kernel that stages blocks in LDS
+        (default), or through the per-run kernel; the outputs are
+        identical."""
         self._check(self.lib.cmi_net_set_tiled(self.h, int(bool(on))))
 
     def input_mode(self):

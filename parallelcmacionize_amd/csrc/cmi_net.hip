@@ -3,32 +3,33 @@
 // first-pass photoionization rate) to the logit of the converged neutral
 // fraction.  Trained and run on the GPU by the kernels below:
 //
-//   conv3_kernel   implicit-GEMM 3-D convolution on BF16 MFMA
-//                  (v_mfma_f32_16x16x32_bf16, FP32 accumulation): one wave
-//                  computes 16 voxels (a run along the last axis) x 16 or 32
-//                  output channels; K = 27 taps x 32 input channels, one MFMA
-//                  per tap and output block.  Serves the forward pass
-//                  (weights [tap][cout][cin], bias, ReLU) and the input
-//                  gradient (the same convolution over the output gradient
-//                  with the flipped, transposed weights, masked by the ReLU of
-//                  the layer below).
-//   wgrad_kernel   weight gradient dW[tap][cout][cin] = sum_v dy[v][cout] *
-//                  x[v + tap][cin] on the same MFMA, K = 32 voxels per
-//                  instruction; FP32 accumulation, one atomic add per weight
-//                  per wave.
-//   plus the loss (mean squared error on logits), bias gradients, Adam on
-//   FP32 master weights, weight packing to BF16, crop sampling and input
-//   normalisation.
+//   conv_block_kernel   implicit-GEMM 3-D convolution on BF16 MFMA
+//                  (v_mfma_f32_16x16x32_bf16, FP32 accumulation) over 8^3
+//                  blocks of a dilation sub-lattice staged in LDS.  Serves the
+//                  forward pass (weights [tap][cout][cin], bias, ReLU) and the
+//                  input gradient (the same convolution over the output
+//                  gradient with the flipped, transposed weights, masked by
+//                  the ReLU of the layer below).
+//   conv3_kernel   the forward convolution without LDS, one wave per run of 16
+//                  voxels (cmi_net_set_tiled(0)): the same outputs bit for bit.
+//   wgrad_block_kernel  weight and bias gradient dW[tap][cout][cin] = sum_v
+//                  dy[v][cout] * x[v + tap][cin] on the same MFMA, K = voxels,
+//                  all 27 taps of a workgroup's blocks kept in registers.
+//   wgrad_first_kernel, wgrad_last_kernel, dgrad_last_kernel  the layers with
+//                  2 inputs and 1 output, taps as a matrix dimension.
+//   plus the loss (mean squared error on logits), Adam on FP32 master weights
+//   with the packing to BF16, crop sampling and input normalisation.
 //
-// Activations are BF16, channels-last with 32 channels ([B][D][H][W][32]);
-// the first layer's 2 input channels and the last layer's single output are
-// zero-padded to the MFMA shapes.
+// Activations are BF16, channels-last with 32 channels ([B][D][H][W][32]); the
+// network's 2 input channels are stored as [B][D][H][W][2] and the gradient of
+// its single output as [B][D][H][W], and padded to the MFMA shapes in LDS.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
 #include <string.h>
 
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/cmi.h"
@@ -50,18 +51,30 @@ __host__ __device__ constexpr int layer_cout(int l) { return l == kLayers - 1 ? 
 __device__ __forceinline__ float bf2f(__bf16 v) { return (float)v; }
 __device__ __forceinline__ __bf16 f2bf(float v) { return (__bf16)v; }
 
+// A voxel's 2 input channels (packed) as its MFMA operand: channels 8*kg ..
+// 8*kg+7 of 32, zeros beyond the second.
+__device__ __forceinline__ bf16x8 feat_operand(uint32_t two, int kg) {
+  union {
+    uint32_t u[4];
+    bf16x8 v;
+  } f;
+  f.u[0] = kg == 0 ? two : 0u;
+  f.u[1] = f.u[2] = f.u[3] = 0u;
+  return f.v;
+}
+
 // ---------------------------------------------------------------------------
 // 3-D convolution (padding 1) as implicit GEMM on MFMA 16x16x32 BF16.
 // Lane l of a wave: A rows (voxels) l%16, A/B k-group (input channels)
 // 8*(l/16)..+7, B column (output channel) l%16; accumulator rows (voxels)
 // 4*(l/16)..+3, column l%16.
 // ---------------------------------------------------------------------------
-template <int NB>
+// kFeat: x is the network's input, 2 channels per voxel.
+template <int NB, bool kFeat>
 __global__ void __launch_bounds__(256) conv3_kernel(
     const __bf16 *__restrict__ x, const __bf16 *__restrict__ w,
     const float *__restrict__ bias, int nrun, int D, int H, int W, int dil,
-    __bf16 *__restrict__ y, float *__restrict__ yf,
-    const __bf16 *__restrict__ mask, int relu) {
+    __bf16 *__restrict__ y, float *__restrict__ yf, int relu) {
   const int lane = threadIdx.x & 63;
   const int run = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (run >= nrun) return;  // whole wave leaves together
@@ -89,7 +102,10 @@ __global__ void __launch_bounds__(256) conv3_kernel(
     if ((unsigned)zd < (unsigned)D && (unsigned)zh < (unsigned)H &&
         (unsigned)zw < (unsigned)W) {
       const size_t vox = (((size_t)b * D + zd) * H + zh) * W + zw;
-      a = *reinterpret_cast<const bf16x8 *>(x + vox * kC + 8 * kg);
+      if (kFeat)
+        a = feat_operand(reinterpret_cast<const uint32_t *>(x)[vox], kg);
+      else
+        a = *reinterpret_cast<const bf16x8 *>(x + vox * kC + 8 * kg);
     } else {
       a = bf16x8{};
     }
@@ -108,7 +124,6 @@ __global__ void __launch_bounds__(256) conv3_kernel(
     for (int i = 0; i < 4; ++i) {
       const size_t v = vbase + 4 * kg + i;
       float r = acc[nb][i] + (bias ? bias[co] : 0.f);
-      if (mask) r = bf2f(mask[v * kC + co]) > 0.f ? r : 0.f;
       if (relu) r = fmaxf(r, 0.f);
       if (y) y[v * kC + co] = f2bf(r);
       if (yf && co == 0) yf[v] = r;
@@ -117,334 +132,785 @@ __global__ void __launch_bounds__(256) conv3_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Tiled forward convolution, for the shapes it divides: the same outputs as
-// conv3_kernel bit for bit (every output voxel's 27 taps go through the same
-// MFMAs with the same operands in the same order).  A convolution with
-// dilation d is d^3 ordinary 3x3x3 convolutions on the sub-lattices of voxels
-// with equal coordinates mod d.  A workgroup takes a block of one sub-lattice,
-// kTZ x kTY runs of 16 voxels along the last axis, and stages the block with
-// its one-voxel halo in LDS, so that each input voxel is read from memory
-// once per block instead of once per tap and output run; each wave computes
-// kRunsPerWave runs and loads each tap's weights once for all of them.
+// Blocks.  A convolution with dilation d is d^3 ordinary 3x3x3 convolutions on
+// the sub-lattices of voxels with equal coordinates mod d.  A workgroup takes a
+// block of one sub-lattice, kBZ x 8 x 8 voxels, and stages it with its
+// one-voxel halo in LDS, so that each input voxel is read from memory once per
+// block instead of once per tap.  Any volume and dilation: a block may reach
+// past its sub-lattice (zeros in, nothing out).  8^3 rather than rows of 16
+// voxels along the last axis, because the sub-lattices of the 64^3 training
+// crops at dilation 8 are 8^3.
 // ---------------------------------------------------------------------------
-constexpr int kTZ = 4, kTY = 8;
-constexpr int kTiledWaves = 4;
-constexpr int kRunsPerWave = kTZ * kTY / kTiledWaves;
-constexpr int kHZ = kTZ + 2, kHY = kTY + 2, kHX = 16 + 2;  // block + halo (voxels)
+constexpr int kE = 8;        // block edge
+constexpr int kHE = kE + 2;  // with the halo
 
-__host__ __device__ inline bool tiled_shape_ok(int D, int H, int W, int dil) {
-  return dil >= 1 && W % (16 * dil) == 0 && H % (kTY * dil) == 0 && D % (kTZ * dil) == 0;
+struct BlockGeo {
+  int D, H, W, dil;
+  int nrz, nry, nrx;  // residues per axis
+  int nbz, nby, nbx;  // blocks per axis of the largest sub-lattice
+  int nblocks;
+};
+
+// One block: its sample, residues, first voxel and sub-lattice extents.
+struct Block {
+  int b, rz, ry, rx, z0, y0, x0, Ds, Hs, Ws;
+};
+
+template <int kBZ>
+__device__ __forceinline__ Block block_of(const BlockGeo &G, int t) {
+  Block k;
+  k.x0 = (t % G.nbx) * kE;
+  t /= G.nbx;
+  k.y0 = (t % G.nby) * kE;
+  t /= G.nby;
+  k.z0 = (t % G.nbz) * kBZ;
+  t /= G.nbz;
+  k.rx = t % G.nrx;
+  t /= G.nrx;
+  k.ry = t % G.nry;
+  t /= G.nry;
+  k.rz = t % G.nrz;
+  k.b = t / G.nrz;
+  k.Ds = (G.D - k.rz + G.dil - 1) / G.dil;
+  k.Hs = (G.H - k.ry + G.dil - 1) / G.dil;
+  k.Ws = (G.W - k.rx + G.dil - 1) / G.dil;
+  return k;
 }
 
-template <int NB>
-__global__ void __launch_bounds__(64 * kTiledWaves) conv3_tiled_kernel(
-    const __bf16 *__restrict__ x, const __bf16 *__restrict__ w,
-    const float *__restrict__ bias, int D, int H, int W, int dil,
-    __bf16 *__restrict__ y, float *__restrict__ yf, int relu) {
-  __shared__ __align__(16) __bf16 blk[kHZ * kHY * kHX * kC];
-  const int Ds = D / dil, Hs = H / dil, Ws = W / dil;  // sub-lattice extents
-  const int nbz = Ds / kTZ, nby = Hs / kTY, nbx = Ws / 16;
-  int t = blockIdx.x;
-  const int bx = t % nbx;
-  t /= nbx;
-  const int by = t % nby;
-  t /= nby;
-  const int bz = t % nbz;
-  t /= nbz;
-  const int rx = t % dil;
-  t /= dil;
-  const int ry = t % dil;
-  t /= dil;
-  const int rz = t % dil;
-  const int b = t / dil;
-  // the block with its halo, in sub-lattice coordinates from (z0, y0, x0);
-  // out of the volume is the zero padding of conv3_kernel
-  const int z0 = bz * kTZ - 1, y0 = by * kTY - 1, x0 = bx * 16 - 1;
+// Voxel number of sub-lattice voxel (sz, sy, sx), or -1 outside the volume.
+__device__ __forceinline__ long long block_voxel(const BlockGeo &G, const Block &k, int sz,
+                                                 int sy, int sx) {
+  if ((unsigned)sz >= (unsigned)k.Ds || (unsigned)sy >= (unsigned)k.Hs ||
+      (unsigned)sx >= (unsigned)k.Ws)
+    return -1;
+  return ((long long)(k.b * G.D + k.rz + G.dil * sz) * G.H + k.ry + G.dil * sy) * G.W + k.rx +
+         G.dil * sx;
+}
+// Halo voxel v (of (kBZ + 2) x 10 x 10) and inner voxel o (of kBZ x 8 x 8).
+__device__ __forceinline__ long long halo_voxel(const BlockGeo &G, const Block &k, int v) {
+  return block_voxel(G, k, k.z0 - 1 + v / (kHE * kHE), k.y0 - 1 + (v / kHE) % kHE,
+                     k.x0 - 1 + v % kHE);
+}
+__device__ __forceinline__ long long inner_voxel(const BlockGeo &G, const Block &k, int o) {
+  return block_voxel(G, k, k.z0 + (o >> 6), k.y0 + ((o >> 3) & 7), k.x0 + (o & 7));
+}
+
+// ---------------------------------------------------------------------------
+// Convolution over 8^3 blocks: the same outputs as conv3_kernel bit for bit
+// (every output voxel's 27 taps go through the same MFMAs with the same
+// operands in the same order).  A wave computes two rows of 8 voxels in each
+// of the block's planes, 8 MFMA rows of 16 voxels, and loads the weights of
+// three taps at a time, one group ahead, once for all of them; 32-channel
+// outputs leave through LDS in 16-byte pieces.  An LDS read of 16 B per lane
+// feeds NB MFMAs, which puts the LDS at the pace of the matrix cores for NB =
+// 2; two workgroups a CU (64 KB of LDS each) overlap one's loads with the
+// other's products.  2^20 voxels (4 crops of 64^3), 32 -> 32 channels: 77 us
+// (63 without the block's loads, 50 without its products), 87 for the rows of
+// 16 voxels it replaces where those divided the volume and 290 for the per-run
+// kernel that the other volumes and the input gradient took.
+// mask: outputs of voxels and channels where it is not positive become 0 (the
+// ReLU of the layer below, for the input gradient).
+// ---------------------------------------------------------------------------
+constexpr int kConvThreads = 256;
+
+template <int NB, bool kFeat>
+__global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
+    BlockGeo G, const __bf16 *__restrict__ x, const __bf16 *__restrict__ w,
+    const float *__restrict__ bias, __bf16 *__restrict__ y, float *__restrict__ yf,
+    const __bf16 *__restrict__ mask, int relu) {
+  constexpr int kHalo = kHE * kHE * kHE;
+  constexpr int kInBytes = kHalo * (kFeat ? 4 : 64);
+  constexpr int kOutBytes = NB == 2 ? kE * kE * kE * 64 : 0;
+  __shared__ __align__(16) unsigned char lds[kInBytes > kOutBytes ? kInBytes : kOutBytes];
+  const Block k = block_of<kE>(G, blockIdx.x);
+  if (k.z0 >= k.Ds || k.y0 >= k.Hs || k.x0 >= k.Ws) return;
   // every thread issues all of its loads before its first LDS store, so the
   // block's memory latency is paid once, not once per load
-  constexpr int kQuarters = kHZ * kHY * kHX * 4;
-  constexpr int kThreadsT = 64 * kTiledWaves;
-  constexpr int kLoads = (kQuarters + kThreadsT - 1) / kThreadsT;
-  bf16x8 vals[kLoads];
+  if (kFeat) {
+    constexpr int kLoads = (kHalo + kConvThreads - 1) / kConvThreads;
+    uint32_t vals[kLoads];
 #pragma unroll
-  for (int k = 0; k < kLoads; ++k) {
-    const int i = (int)threadIdx.x + k * kThreadsT;
-    vals[k] = bf16x8{};
-    if (i < kQuarters) {
-      const int q = i & 3;  // 16-byte quarter of the voxel's 32 channels
-      const int v = i >> 2;
-      const int hx = v % kHX, hy = (v / kHX) % kHY, hz = v / (kHX * kHY);
-      const int sz = z0 + hz, sy = y0 + hy, sx = x0 + hx;
-      if ((unsigned)sz < (unsigned)Ds && (unsigned)sy < (unsigned)Hs &&
-          (unsigned)sx < (unsigned)Ws) {
-        const size_t vox = (((size_t)b * D + (rz + dil * sz)) * H + (ry + dil * sy)) * W +
-                           (rx + dil * sx);
-        vals[k] = *reinterpret_cast<const bf16x8 *>(x + vox * kC + 8 * q);
-      }
+    for (int i = 0; i < kLoads; ++i) {
+      const int v = (int)threadIdx.x + i * kConvThreads;
+      const long long g = v < kHalo ? halo_voxel(G, k, v) : -1;
+      vals[i] = g >= 0 ? reinterpret_cast<const uint32_t *>(x)[g] : 0u;
     }
-  }
 #pragma unroll
-  for (int k = 0; k < kLoads; ++k) {
-    const int i = (int)threadIdx.x + k * kThreadsT;
-    if (i < kQuarters) *reinterpret_cast<bf16x8 *>(blk + (size_t)i * 8) = vals[k];
+    for (int i = 0; i < kLoads; ++i) {
+      const int v = (int)threadIdx.x + i * kConvThreads;
+      if (v < kHalo) reinterpret_cast<uint32_t *>(lds)[v] = vals[i];
+    }
+  } else {
+    constexpr int kLoads = (4 * kHalo + kConvThreads - 1) / kConvThreads;
+    bf16x8 vals[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int p = (int)threadIdx.x + i * kConvThreads;  // 16-byte piece
+      const long long g = p < 4 * kHalo ? halo_voxel(G, k, p >> 2) : -1;
+      vals[i] = bf16x8{};
+      if (g >= 0) vals[i] = *reinterpret_cast<const bf16x8 *>(x + g * kC + 8 * (p & 3));
+    }
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      const int p = (int)threadIdx.x + i * kConvThreads;
+      if (p < 4 * kHalo) reinterpret_cast<bf16x8 *>(lds)[p] = vals[i];
+    }
   }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int vl = lane & 15;  // voxel (A row) / output channel (B column)
   const int kg = lane >> 4;  // k group: channels 8*kg .. 8*kg+7
   const int NOUT = 16 * NB;
-  f32x4 acc[kRunsPerWave][NB];
+  const int first = (2 * wave + (vl >> 3)) * kHE + (vl & 7);  // halo voxel of tap 0
+  const int nz = min(kE, k.Ds - k.z0);
+  const bool rows = 2 * wave < k.Hs - k.y0;  // the wave has voxels
+  f32x4 acc[kE][NB];
 #pragma unroll
-  for (int r = 0; r < kRunsPerWave; ++r)
+  for (int r = 0; r < kE; ++r)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[r][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // each tap's weights are loaded one tap ahead
-  bf16x8 bw[NB], bn[NB];
+  auto products = [&](auto whole) {
+    bf16x8 bw[3][NB], bn[3][NB];
+    auto load_weights = [&](int group) {
 #pragma unroll
-  for (int nb = 0; nb < NB; ++nb)
-    bn[nb] = *reinterpret_cast<const bf16x8 *>(w + ((size_t)nb * 16 + vl) * kC + 8 * kg);
+      for (int kw = 0; kw < 3; ++kw)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          bn[kw][nb] = *reinterpret_cast<const bf16x8 *>(
+              w + ((size_t)(3 * group + kw) * NOUT + nb * 16 + vl) * kC + 8 * kg);
+    };
+    load_weights(0);
 #pragma unroll 1
-  for (int tap = 0; tap < kTaps; ++tap) {
-    const int kd = tap / 9, kh = (tap / 3) % 3, kw = tap % 3;
+    for (int group = 0; group < 9; ++group) {
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) bw[nb] = bn[nb];
-    if (tap + 1 < kTaps) {
+      for (int kw = 0; kw < 3; ++kw)
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-        bn[nb] = *reinterpret_cast<const bf16x8 *>(
-            w + ((size_t)(tap + 1) * NOUT + nb * 16 + vl) * kC + 8 * kg);
-    }
+        for (int nb = 0; nb < NB; ++nb) bw[kw][nb] = bn[kw][nb];
+      if (group + 1 < 9) load_weights(group + 1);
+      const int at = first + ((group / 3) * kHE + group % 3) * kHE;
 #pragma unroll
-    for (int r = 0; r < kRunsPerWave; ++r) {
-      const int j = wave * kRunsPerWave + r;
-      const int jz = j / kTY, jy = j % kTY;
-      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(
-          blk + ((size_t)((jz + kd) * kHY + (jy + kh)) * kHX + (vl + kw)) * kC + 8 * kg);
+      for (int kw = 0; kw < 3; ++kw) {
 #pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-        acc[r][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[nb], acc[r][nb], 0, 0, 0);
-    }
-  }
-  if (NB == 2 && y && !yf) {
-    // 32-channel output: through the (now free) LDS block as [run][16
-    // voxels][32 channels], then written out in 16-byte pieces, a voxel's
-    // 64 bytes by 4 neighbouring lanes
-    __syncthreads();
+        for (int r = 0; r < kE; ++r) {
+          if (!decltype(whole)::value && r >= nz) break;
+          const int v = at + kw + r * kHE * kHE;
+          bf16x8 a;
+          if (kFeat)
+            a = feat_operand(reinterpret_cast<const uint32_t *>(lds)[v], kg);
+          else
+            a = *reinterpret_cast<const bf16x8 *>(lds + (size_t)v * 64 + 16 * kg);
 #pragma unroll
-    for (int r = 0; r < kRunsPerWave; ++r) {
-      const int j = wave * kRunsPerWave + r;
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        const int co = nb * 16 + vl;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float o = acc[r][nb][i] + (bias ? bias[co] : 0.f);
-          if (relu) o = fmaxf(o, 0.f);
-          blk[((size_t)j * 16 + 4 * kg + i) * kC + co] = f2bf(o);
+          for (int nb = 0; nb < NB; ++nb)
+            acc[r][nb] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw[kw][nb], acc[r][nb], 0, 0, 0);
         }
       }
     }
-    __syncthreads();
-    constexpr int kOut = kTZ * kTY * 16 * 4;  // 16-byte pieces of the block's outputs
-#pragma unroll
-    for (int k = 0; k < kOut / kThreadsT; ++k) {
-      const int i = (int)threadIdx.x + k * kThreadsT;
-      const int q = i & 3, vx = (i >> 2) & 15, j = i >> 6;
-      const int gz = rz + dil * (bz * kTZ + (j / kTY)), gy = ry + dil * (by * kTY + (j % kTY));
-      const size_t v = (((size_t)b * D + gz) * H + gy) * W + rx + dil * (bx * 16 + vx);
-      *reinterpret_cast<bf16x8 *>(y + v * kC + 8 * q) =
-          *reinterpret_cast<const bf16x8 *>(blk + (size_t)i * 8);
-    }
-    return;
+  };
+  if (rows) {
+    if (nz == kE)
+      products(std::true_type{});
+    else
+      products(std::false_type{});
   }
+  if (NB == 2) {
+    // through the (now free) LDS block as [voxel][32 channels]
+    __bf16 *out = reinterpret_cast<__bf16 *>(lds);
+    __syncthreads();
 #pragma unroll
-  for (int r = 0; r < kRunsPerWave; ++r) {
-    const int j = wave * kRunsPerWave + r;
-    const int gz = rz + dil * (bz * kTZ + (j / kTY)), gy = ry + dil * (by * kTY + (j % kTY));
-    const size_t row = (((size_t)b * D + gz) * H + gy) * W;
+    for (int r = 0; r < kE; ++r)
 #pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const int co = nb * 16 + vl;
+      for (int nb = 0; nb < NB; ++nb) {
+        const int co = nb * 16 + vl;
+        const float add = bias ? bias[co] : 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int vrow = 4 * kg + i;
+          float o = acc[r][nb][i] + add;
+          if (relu) o = fmaxf(o, 0.f);
+          out[((r * kE + 2 * wave + (vrow >> 3)) * kE + (vrow & 7)) * kC + co] = f2bf(o);
+        }
+      }
+    __syncthreads();
+    constexpr int kOut = kE * kE * kE * 4 / kConvThreads;  // 16-byte pieces per thread
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) {
+      const int p = (int)threadIdx.x + i * kConvThreads;
+      const long long g = inner_voxel(G, k, p >> 2);
+      if (g < 0) continue;
+      bf16x8 o = reinterpret_cast<const bf16x8 *>(lds)[p];
+      if (mask) {
+        const bf16x8 m = *reinterpret_cast<const bf16x8 *>(mask + g * kC + 8 * (p & 3));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = bf2f(m[e]) > 0.f ? o[e] : f2bf(0.f);
+      }
+      *reinterpret_cast<bf16x8 *>(y + g * kC + 8 * (p & 3)) = o;
+    }
+  } else if (vl == 0) {
+    // the network's output: channel 0 only
+#pragma unroll
+    for (int r = 0; r < kE; ++r)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const size_t v = row + rx + dil * (bx * 16 + 4 * kg + i);
-        float o = acc[r][nb][i] + (bias ? bias[co] : 0.f);
-        if (relu) o = fmaxf(o, 0.f);
-        if (y) y[v * kC + co] = f2bf(o);
-        if (yf && co == 0) yf[v] = o;
+        const int vrow = 4 * kg + i;
+        const long long g = block_voxel(G, k, k.z0 + r, k.y0 + 2 * wave + (vrow >> 3),
+                                        k.x0 + (vrow & 7));
+        if (g >= 0) yf[g] = acc[r][0][i] + (bias ? bias[0] : 0.f);
       }
-    }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Weight gradient: dW[tap][cout][cin] += sum over voxels of
-// dy[v][cout] * x[v + tap - 1][cin].  A wave owns (tap, cout block) and both
-// cin blocks and sweeps `rows_per_wave` runs of 32 voxels.
+// Weight gradients.  K of the MFMA runs over voxels, so both operands are
+// columns of channels-last data: the LDS transpose read (ds_read_b64_tr_b16,
+// 4 voxels x 16 channels per 16 lanes) forms them, two reads for the 8
+// consecutive voxels of a lane.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) wgrad_kernel(
-    const __bf16 *__restrict__ dy, const __bf16 *__restrict__ x, int nb_out,
-    int nrow, int rows_per_wave, int D, int H, int W, int dil,
-    float *__restrict__ dW, int NOUT) {
-  const int lane = threadIdx.x & 63;
-  const int wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int nchunks = (nrow + rows_per_wave - 1) / rows_per_wave;
-  const int job = wave;
-  if (job >= kTaps * nb_out * nchunks) return;
-  const int chunk = job % nchunks;
-  const int mb = (job / nchunks) % nb_out;
-  const int tap = job / (nchunks * nb_out);
-  const int kd = tap / 9, kh = (tap / 3) % 3, kw = tap % 3;
-  const int ml = lane & 15;   // A row: cout; B column: cin
-  const int kg = lane >> 4;   // voxels 8*kg .. 8*kg+7 of the 32-voxel run
-  f32x4 acc0 = f32x4{0.f, 0.f, 0.f, 0.f}, acc1 = acc0;
-  const int wr = W >> 5;
-  const int r0 = chunk * rows_per_wave, r1 = min(nrow, r0 + rows_per_wave);
-  for (int row = r0; row < r1; ++row) {
-    int t = row;
-    const int w0 = (t % wr) << 5;
-    t /= wr;
-    const int h = t % H;
-    t /= H;
-    const int d = t % D;
-    const int b = t / D;
-    const size_t vbase = (((size_t)b * D + d) * H + h) * W + w0 + 8 * kg;
-    bf16x8 a, b0, b1;
-    const int zd = d + (kd - 1) * dil, zh = h + (kh - 1) * dil;
-    const bool rowin = (unsigned)zd < (unsigned)D && (unsigned)zh < (unsigned)H;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+union Operand {
+  s16x4 h[2];
+  bf16x8 v;
+};
+
+// p: the lane's share of voxels x .. x+3 (its voxel (lane % 16) / 4, channels
+// 4 (lane % 4) ..); step: elements from voxel x to voxel x+4.
+__device__ __forceinline__ bf16x8 voxels_operand(const __bf16 *p, int step) {
+  Operand o;
+  o.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4 *)p);
+  o.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4 *)(p + step));
+  return o.v;
+}
+
+// Workgroups add their sums into kCopies copies of the gradient in turn
+// (grad_copy), which the optimiser sums up.  Adds of many workgroups to one
+// cache line pass one at a time: 512 workgroups on one copy cost 35 to 42 us
+// of a 32-channel layer's 125, on 16 copies 2 to 3.
+constexpr int kCopies = 16;
+__device__ __forceinline__ float *grad_copy(float *g, size_t stride) {
+  return g + (blockIdx.x % kCopies) * stride;
+}
+
+constexpr int kGZ = 4;  // planes of a weight-gradient block
+constexpr int kGVox = kGZ * kE * kE;
+constexpr int kGHalo = (kGZ + 2) * kHE * kHE;
+constexpr int kGThreads = 256;
+constexpr int kTapsPerWave = 7;
+
+// The 32 -> 32 channel layers.  A wave owns 7 taps (the last wave 6 and the
+// bias, whose second operand is ones) and keeps their 32 x 32 gradients in
+// registers over all blocks of its workgroup; one FP32 atomic add per weight
+// and workgroup at the end.  Per 32 voxels a wave reads 32 operand halves
+// from LDS for 28 MFMAs, so LDS and matrix cores are about level; the next
+// block's loads are in flight under them.  2^20 voxels: 100 us (16 of them the
+// final adds; 76 with an eighth of the products), against 970 for one wave per
+// tap, channel block and 16 runs with 2-byte operand loads.
+__global__ void __launch_bounds__(kGThreads, 2) wgrad_block_kernel(
+    BlockGeo G, const __bf16 *__restrict__ dy, const __bf16 *__restrict__ x,
+    float *__restrict__ grad, size_t stride, size_t off_w, size_t off_b) {
+  float *const dW = grad_copy(grad, stride) + off_w, *const db = grad_copy(grad, stride) + off_b;
+  __shared__ __align__(16) __bf16 xs[kGHalo * kC];
+  __shared__ __align__(16) __bf16 ds[kGVox * kC];
+  constexpr int kXL = (4 * kGHalo + kGThreads - 1) / kGThreads, kDL = 4 * kGVox / kGThreads;
+  bf16x8 px[kXL], pd[kDL];
+  auto load = [&](int blk) {
+    const Block k = block_of<kGZ>(G, blk);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      a[j] = dy[(vbase + j) * kC + mb * 16 + ml];
-      const int zw = w0 + 8 * kg + j + (kw - 1) * dil;
-      if (rowin && (unsigned)zw < (unsigned)W) {
-        const size_t vx = (((size_t)b * D + zd) * H + zh) * W + zw;
-        b0[j] = x[vx * kC + ml];
-        b1[j] = x[vx * kC + 16 + ml];
-      } else {
-        b0[j] = (__bf16)0.f;
-        b1[j] = (__bf16)0.f;
+    for (int i = 0; i < kXL; ++i) {
+      const int p = (int)threadIdx.x + i * kGThreads;
+      const long long g = p < 4 * kGHalo ? halo_voxel(G, k, p >> 2) : -1;
+      px[i] = bf16x8{};
+      if (g >= 0) px[i] = *reinterpret_cast<const bf16x8 *>(x + g * kC + 8 * (p & 3));
+    }
+#pragma unroll
+    for (int i = 0; i < kDL; ++i) {
+      const int p = (int)threadIdx.x + i * kGThreads;
+      const long long g = inner_voxel(G, k, p >> 2);
+      pd[i] = bf16x8{};
+      if (g >= 0) pd[i] = *reinterpret_cast<const bf16x8 *>(dy + g * kC + 8 * (p & 3));
+    }
+  };
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int ml = lane & 15, kg = lane >> 4, r4 = ml >> 2, c4 = lane & 3;
+  const __bf16 *const dl = ds + ((kg * kE + r4) * kC + 4 * c4);
+  const __bf16 *const xl = xs + ((kg * kHE + r4) * kC + 4 * c4);
+  bf16x8 ones;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) ones[j] = f2bf(1.f);
+  f32x4 acc[kTapsPerWave][2][2];
+#pragma unroll
+  for (int t = 0; t < kTapsPerWave; ++t)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[t][q >> 1][q & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int blk = blockIdx.x;
+  if (blk < G.nblocks) load(blk);
+  for (; blk < G.nblocks; blk += gridDim.x) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kXL; ++i) {
+      const int p = (int)threadIdx.x + i * kGThreads;
+      if (p < 4 * kGHalo) reinterpret_cast<bf16x8 *>(xs)[p] = px[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kDL; ++i)
+      reinterpret_cast<bf16x8 *>(ds)[threadIdx.x + i * kGThreads] = pd[i];
+    __syncthreads();
+    if (blk + (int)gridDim.x < G.nblocks) load(blk + gridDim.x);
+    // 32 voxels at a time: 4 rows of 8, row kg the lane's
+#pragma unroll 1
+    for (int s = 0; s < kGVox / 32; ++s) {
+      const __bf16 *const dp = dl + s * (4 * kE) * kC;
+      const __bf16 *const xp = xl + ((s >> 1) * kHE * kHE + (s & 1) * 4 * kHE) * kC;
+      bf16x8 a[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) a[m] = voxels_operand(dp + 16 * m, 4 * kC);
+#pragma unroll
+      for (int t = 0; t < kTapsPerWave; ++t) {
+        const int tap = wave * kTapsPerWave + t;
+        if (t + 1 < kTapsPerWave || tap < kTaps) {
+          const int off = ((tap / 9) * kHE + (tap / 3) % 3) * kHE + tap % 3;
+#pragma unroll
+          for (int n = 0; n < 2; ++n) {
+            const bf16x8 b = voxels_operand(xp + off * kC + 16 * n, 4 * kC);
+#pragma unroll
+            for (int m = 0; m < 2; ++m)
+              acc[t][m][n] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b, acc[t][m][n], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int m = 0; m < 2; ++m)
+            acc[t][m][0] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], ones, acc[t][m][0], 0, 0, 0);
+        }
       }
     }
-    acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b0, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b1, acc1, 0, 0, 0);
   }
   // accumulator: rows (cout) 4*kg..+3, column (cin) ml
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int co = mb * 16 + 4 * kg + i;
-    atomicAdd(&dW[((size_t)tap * NOUT + co) * kC + ml], acc0[i]);
-    atomicAdd(&dW[((size_t)tap * NOUT + co) * kC + 16 + ml], acc1[i]);
+  for (int t = 0; t < kTapsPerWave; ++t) {
+    const int tap = wave * kTapsPerWave + t;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int co = 16 * m + 4 * kg + i;
+        if (tap < kTaps) {
+          atomicAdd(&dW[((size_t)tap * kC + co) * kC + ml], acc[t][m][0][i]);
+          atomicAdd(&dW[((size_t)tap * kC + co) * kC + 16 + ml], acc[t][m][1][i]);
+        } else if (ml == 0) {
+          atomicAdd(&db[co], acc[t][m][0][i]);
+        }
+      }
   }
 }
 
-// db[c] += sum over voxels of dy[v][c], c < nc
-__global__ void bgrad_kernel(const __bf16 *__restrict__ dy, size_t nvox, int nc,
-                             float *__restrict__ db) {
-  __shared__ float sh[kC];
-  if (threadIdx.x < kC) sh[threadIdx.x] = 0.f;
-  __syncthreads();
-  const int c = threadIdx.x & 31;
-  float s = 0.f;
-  if (c < nc) {
-    for (size_t v = (size_t)blockIdx.x * (blockDim.x >> 5) + (threadIdx.x >> 5); v < nvox;
-         v += (size_t)gridDim.x * (blockDim.x >> 5))
-      s += bf2f(dy[v * kC + c]);
-    atomicAdd(&sh[c], s);
+// The first layer (2 input channels): tap and input channel together are the
+// MFMA's columns, 54 of 64 (16 to a wave), with the bias (ones) as column 54.
+// The input is staged as planes shifted by each tap of the last axis, so that
+// an operand's 8 voxels are one aligned read.  Bound by reading dy once and
+// the final adds (42 us for 2^20 voxels; 59 with twice the workgroups).
+__global__ void __launch_bounds__(kGThreads) wgrad_first_kernel(
+    BlockGeo G, const __bf16 *__restrict__ dy, const uint32_t *__restrict__ feat,
+    float *__restrict__ grad, size_t stride, size_t off_w, size_t off_b) {
+  float *const dW = grad_copy(grad, stride) + off_w, *const db = grad_copy(grad, stride) + off_b;
+  constexpr int kPlane = (kGZ + 2) * kHE * kE;  // one channel, one shift
+  __shared__ __align__(16) __bf16 ds[kGVox * kC];
+  __shared__ __align__(16) uint16_t pl[3 * 2 * kPlane];
+  constexpr int kFL = (kGHalo + kGThreads - 1) / kGThreads, kDL = 4 * kGVox / kGThreads;
+  uint32_t pf[kFL];
+  bf16x8 pd[kDL];
+  auto load = [&](int blk) {
+    const Block k = block_of<kGZ>(G, blk);
+#pragma unroll
+    for (int i = 0; i < kFL; ++i) {
+      const int v = (int)threadIdx.x + i * kGThreads;
+      const long long g = v < kGHalo ? halo_voxel(G, k, v) : -1;
+      pf[i] = g >= 0 ? feat[g] : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < kDL; ++i) {
+      const int p = (int)threadIdx.x + i * kGThreads;
+      const long long g = inner_voxel(G, k, p >> 2);
+      pd[i] = bf16x8{};
+      if (g >= 0) pd[i] = *reinterpret_cast<const bf16x8 *>(dy + g * kC + 8 * (p & 3));
+    }
+  };
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ml = lane & 15, kg = lane >> 4, r4 = ml >> 2, c4 = lane & 3;
+  const __bf16 *const dl = ds + ((kg * kE + r4) * kC + 4 * c4);
+  const int n = 16 * wave + ml, tap = n >> 1, c = n & 1;
+  const bool real = tap < kTaps;
+  const uint16_t *const fl =
+      pl + (real ? (((tap % 3) * 2 + c) * kPlane + ((tap / 9) * kHE + (tap / 3) % 3) * kE) : 0) +
+      kg * kE;
+  bf16x8 fixed;  // the operand of a column that is no tap
+#pragma unroll
+  for (int j = 0; j < 8; ++j) fixed[j] = f2bf(n == 2 * kTaps ? 1.f : 0.f);
+  f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+  int blk = blockIdx.x;
+  if (blk < G.nblocks) load(blk);
+  for (; blk < G.nblocks; blk += gridDim.x) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kFL; ++i) {
+      const int v = (int)threadIdx.x + i * kGThreads;
+      const int hx = v % kHE, row = v / kHE;
+      if (v < kGHalo) {
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+          if ((unsigned)(hx - s) < (unsigned)kE) {
+            pl[(2 * s) * kPlane + row * kE + hx - s] = (uint16_t)pf[i];
+            pl[(2 * s + 1) * kPlane + row * kE + hx - s] = (uint16_t)(pf[i] >> 16);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kDL; ++i)
+      reinterpret_cast<bf16x8 *>(ds)[threadIdx.x + i * kGThreads] = pd[i];
+    __syncthreads();
+    if (blk + (int)gridDim.x < G.nblocks) load(blk + gridDim.x);
+#pragma unroll
+    for (int s = 0; s < kGVox / 32; ++s) {
+      bf16x8 b = *reinterpret_cast<const bf16x8 *>(
+          fl + ((s >> 1) * kHE + (s & 1) * 4) * kE);
+      if (!real) b = fixed;
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const bf16x8 a = voxels_operand(dl + s * (4 * kE) * kC + 16 * m, 4 * kC);
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[m], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int co = 16 * m + 4 * kg + i;
+      if (real)
+        atomicAdd(&dW[((size_t)tap * kC + co) * kC + c], acc[m][i]);
+      else if (n == 2 * kTaps)
+        atomicAdd(&db[co], acc[m][i]);
+    }
+}
+
+// The last layer (1 output channel): the taps are the MFMA's rows, dW[tap][ci]
+// = sum_u dz[u - tap] x[u][ci], with the output gradient dz (one value per
+// voxel) staged in shifted planes.  Bound by reading x once (28 us for 2^20
+// voxels).  (The bias gradient, the sum of dz, comes with the loss.)
+__global__ void __launch_bounds__(kGThreads) wgrad_last_kernel(
+    BlockGeo G, const uint16_t *__restrict__ dz, const __bf16 *__restrict__ x,
+    float *__restrict__ grad, size_t stride, size_t off_w, int NOUT) {
+  float *const dW = grad_copy(grad, stride) + off_w;
+  constexpr int kPlane = (kGZ + 2) * kHE * kE;
+  __shared__ __align__(16) __bf16 xs[kGVox * kC];
+  __shared__ __align__(16) uint16_t pl[3 * kPlane];
+  constexpr int kFL = (kGHalo + kGThreads - 1) / kGThreads, kDL = 4 * kGVox / kGThreads;
+  uint16_t pz[kFL];
+  bf16x8 px[kDL];
+  auto load = [&](int blk) {
+    const Block k = block_of<kGZ>(G, blk);
+#pragma unroll
+    for (int i = 0; i < kFL; ++i) {
+      const int v = (int)threadIdx.x + i * kGThreads;
+      const long long g = v < kGHalo ? halo_voxel(G, k, v) : -1;
+      pz[i] = g >= 0 ? dz[g] : (uint16_t)0;
+    }
+#pragma unroll
+    for (int i = 0; i < kDL; ++i) {
+      const int p = (int)threadIdx.x + i * kGThreads;
+      const long long g = inner_voxel(G, k, p >> 2);
+      px[i] = bf16x8{};
+      if (g >= 0) px[i] = *reinterpret_cast<const bf16x8 *>(x + g * kC + 8 * (p & 3));
+    }
+  };
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int ml = lane & 15, kg = lane >> 4, r4 = ml >> 2, c4 = lane & 3;
+  const __bf16 *const xl = xs + ((kg * kE + r4) * kC + 4 * c4);
+  // the lane's row of either half of the taps: halo offset of u - (tap - 1)
+  const uint16_t *zl[2];
+  bool real[2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int tap = 16 * m + ml;
+    real[m] = tap < kTaps;
+    const int t = real[m] ? tap : 0;
+    zl[m] = pl + (2 - t % 3) * kPlane + ((2 - t / 9) * kHE + 2 - (t / 3) % 3) * kE + kg * kE;
+  }
+  f32x4 acc[2][2];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) acc[q >> 1][q & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int blk = blockIdx.x;
+  if (blk < G.nblocks) load(blk);
+  for (; blk < G.nblocks; blk += gridDim.x) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kFL; ++i) {
+      const int v = (int)threadIdx.x + i * kGThreads;
+      const int hx = v % kHE, row = v / kHE;
+      if (v < kGHalo) {
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+          if ((unsigned)(hx - s) < (unsigned)kE) pl[s * kPlane + row * kE + hx - s] = pz[i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kDL; ++i)
+      reinterpret_cast<bf16x8 *>(xs)[threadIdx.x + i * kGThreads] = px[i];
+    __syncthreads();
+    if (blk + (int)gridDim.x < G.nblocks) load(blk + gridDim.x);
+    // each wave takes two of the block's eight 32-voxel pieces
+#pragma unroll
+    for (int h = 0; h < kGVox / 32 / 4; ++h) {
+      const int s = wave + 4 * h;
+      bf16x8 a[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        a[m] = *reinterpret_cast<const bf16x8 *>(zl[m] + ((s >> 1) * kHE + (s & 1) * 4) * kE);
+        if (!real[m]) a[m] = bf16x8{};
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const bf16x8 b = voxels_operand(xl + s * (4 * kE) * kC + 16 * c, 4 * kC);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          acc[m][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b, acc[m][c], 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int tap = 16 * m + 4 * kg + i;
+      if (tap < kTaps) {
+        atomicAdd(&dW[(size_t)tap * NOUT * kC + ml], acc[m][0][i]);
+        atomicAdd(&dW[(size_t)tap * NOUT * kC + 16 + ml], acc[m][1][i]);
+      }
+    }
+}
+
+// Input gradient of the last layer: dx[v][ci] = sum over taps of dz[v + tap - 1]
+// w[tap][ci], masked by the ReLU of the layer below; the taps are the MFMA's K
+// (27 of 32), one product per 16 voxels and 16 channels.  Bound by the mask
+// read and dx written once: 41 us for 2^20 voxels, 290 through 27 products
+// per 16 voxels of a 32-channel dz.
+__global__ void __launch_bounds__(kConvThreads) dgrad_last_kernel(
+    BlockGeo G, const uint16_t *__restrict__ dz, const __bf16 *__restrict__ wb,
+    const __bf16 *__restrict__ mask, __bf16 *__restrict__ dx) {
+  constexpr int kHalo = kHE * kHE * kHE;
+  __shared__ uint16_t zs[kHalo];
+  __shared__ __align__(16) __bf16 out[kE * kE * kE * kC];
+  const Block k = block_of<kE>(G, blockIdx.x);
+  if (k.z0 >= k.Ds || k.y0 >= k.Hs || k.x0 >= k.Ws) return;
+  constexpr int kLoads = (kHalo + kConvThreads - 1) / kConvThreads;
+  uint16_t vals[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int v = (int)threadIdx.x + i * kConvThreads;
+    const long long g = v < kHalo ? halo_voxel(G, k, v) : -1;
+    vals[i] = g >= 0 ? dz[g] : (uint16_t)0;
+  }
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int v = (int)threadIdx.x + i * kConvThreads;
+    if (v < kHalo) zs[v] = vals[i];
+  }
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int vl = lane & 15, kg = lane >> 4;
+  union Taps {
+    uint16_t u[8];
+    bf16x8 v;
+  };
+  Taps b[2];
+  int off[8];  // halo voxel of the lane's taps at the first plane
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int t = 8 * kg + j;
+    off[j] = (2 * wave + (vl >> 3)) * kHE + (vl & 7);
+    if (t < kTaps) off[j] += ((t / 9) * kHE + (t / 3) % 3) * kHE + t % 3;
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+      b[n].u[j] = t < kTaps ? reinterpret_cast<const uint16_t *>(
+                                  wb)[((size_t)t * 32 + 16 * n + vl) * kC]
+                            : (uint16_t)0;
   }
   __syncthreads();
-  if (threadIdx.x < nc) atomicAdd(&db[threadIdx.x], sh[threadIdx.x]);
+#pragma unroll
+  for (int r = 0; r < kE; ++r) {
+    Taps a;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      a.u[j] = 8 * kg + j < kTaps ? zs[off[j] + r * kHE * kHE] : (uint16_t)0;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, b[n].v, acc, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int vrow = 4 * kg + i;
+        out[((r * kE + 2 * wave + (vrow >> 3)) * kE + (vrow & 7)) * kC + 16 * n + vl] =
+            f2bf(acc[i]);
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kE * kE * kE * 4 / kConvThreads; ++i) {
+    const int p = (int)threadIdx.x + i * kConvThreads;
+    const long long g = inner_voxel(G, k, p >> 2);
+    if (g < 0) continue;
+    bf16x8 o = reinterpret_cast<const bf16x8 *>(out)[p];
+    const bf16x8 m = *reinterpret_cast<const bf16x8 *>(mask + g * kC + 8 * (p & 3));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = bf2f(m[e]) > 0.f ? o[e] : f2bf(0.f);
+    *reinterpret_cast<bf16x8 *>(dx + g * kC + 8 * (p & 3)) = o;
+  }
 }
 
 // Weighted mean squared error on logits: with e = z - t and w = w_pos for
 // e > 0 (a prediction more neutral than the target), 1 otherwise,
-// loss += sum w e^2 / n; dy[v][0] = 2 w e / n, other channels 0.
-__global__ void mse_kernel(const float *__restrict__ z, const float *__restrict__ tgt,
-                           size_t n, float w_pos, __bf16 *__restrict__ dy,
-                           float *__restrict__ loss) {
-  __shared__ float sh[4];
-  float s = 0.f;
+// loss += sum w e^2 / n; dz[v] = 2 w e / n, and its sum to the bias gradient.
+__global__ void __launch_bounds__(256) mse_kernel(
+    const float *__restrict__ z, const float *__restrict__ tgt, size_t n, float w_pos,
+    __bf16 *__restrict__ dz, float *__restrict__ grad, size_t stride, size_t off_loss,
+    size_t off_b) {
+  __shared__ float sh[8];
+  float s = 0.f, d = 0.f;
   const float inv = 1.f / (float)n;
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
        v += (size_t)gridDim.x * blockDim.x) {
     const float e = z[v] - tgt[v];
     const float w = e > 0.f ? w_pos : 1.f;
     s += w * e * e;
-    __bf16 *o = dy + v * kC;
-    o[0] = f2bf(2.f * w * e * inv);
+    const __bf16 g = f2bf(2.f * w * e * inv);
+    dz[v] = g;
+    d += bf2f(g);
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  for (int o = 32; o > 0; o >>= 1) {
+    s += __shfl_xor(s, o, 64);
+    d += __shfl_xor(d, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    sh[threadIdx.x >> 6] = s;
+    sh[4 + (threadIdx.x >> 6)] = d;
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
-    float t = 0.f;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += sh[w];
-    atomicAdd(loss, t * inv);
+    float *const g = grad_copy(grad, stride);
+    atomicAdd(g + off_loss, (sh[0] + sh[1] + sh[2] + sh[3]) * inv);
+    atomicAdd(g + off_b, sh[4] + sh[5] + sh[6] + sh[7]);
   }
 }
 
-// Adam (Kingma & Ba 2015) on FP32 master parameters.
-__global__ void adam_kernel(float *__restrict__ p, const float *__restrict__ g,
+// Layers of the master vector (FP32, padded to the MFMA shapes): W[27][NOUT]
+// [32] (tap, output channel, input channel; entries beyond the real channels
+// stay 0: their gradients are 0) then b[NOUT].  Packed BF16 GEMM weights: fwd
+// = W as is, and the input-gradient weights bwd[t'][cin][cout] =
+// W[26-t'][cout][cin] ([27][32][32], zero for cout >= NOUT).
+struct Layers {
+  size_t off_w[kLayers], off_b[kLayers];
+  int nout[kLayers];
+  __bf16 *fwd[kLayers], *bwd[kLayers];
+};
+
+__global__ void pack_kernel(const float *__restrict__ p, Layers L) {
+  const int n = kTaps * 32 * 32;
+  const int l = blockIdx.y, NOUT = L.nout[l];
+  const float *const master = p + L.off_w[l];
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    const int tap = i / 1024, o = (i / 32) % 32, k = i % 32;
+    if (o < NOUT)
+      L.fwd[l][((size_t)tap * NOUT + o) * kC + k] = f2bf(master[((size_t)tap * NOUT + o) * kC + k]);
+    const float vb = k < NOUT ? master[((size_t)(kTaps - 1 - tap) * NOUT + k) * kC + o] : 0.f;
+    L.bwd[l][((size_t)tap * 32 + o) * kC + k] = f2bf(vb);
+  }
+}
+
+__device__ __forceinline__ float sum_copies(const float *__restrict__ g, size_t stride,
+                                            size_t i) {
+  float s = 0.f;
+#pragma unroll
+  for (int c = 0; c < kCopies; ++c) s += g[c * stride + i];
+  return s;
+}
+
+// The gradient (n values) and the loss after it, summed over the copies.
+__global__ void sum_grad_kernel(const float *__restrict__ g, size_t stride, size_t n,
+                                float *__restrict__ out) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i <= n;
+       i += (size_t)gridDim.x * blockDim.x)
+    out[i] = sum_copies(g, stride, i);
+}
+
+// Adam (Kingma & Ba 2015) on the FP32 master parameters; an updated weight
+// goes to its place in both packed copies at once.  Value n of the gradient is
+// the loss.
+__global__ void adam_kernel(float *__restrict__ p, const float *__restrict__ g, size_t stride,
                             float *__restrict__ m, float *__restrict__ v, size_t n,
                             float lr, float b1, float b2, float eps, float c1,
-                            float c2, float wd) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+                            float c2, float wd, Layers L, float *__restrict__ loss) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i <= n;
        i += (size_t)gridDim.x * blockDim.x) {
-    const float gi = g[i] + wd * p[i];
+    const float gs = sum_copies(g, stride, i);
+    if (i == n) {
+      *loss = gs;
+      continue;
+    }
+    const float gi = gs + wd * p[i];
     const float mi = b1 * m[i] + (1.f - b1) * gi;
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  }
-}
-
-// FP32 master layout of layer l (padded to the MFMA shapes): W[27][NOUT][32]
-// (tap, output channel, input channel; entries beyond the real channels stay
-// 0: their gradients are 0) then b[NOUT].  Packed BF16 GEMM weights: fwd =
-// W as is, and the input-gradient weights bwd[t'][cin][cout] = W[26-t'][cout]
-// [cin] ([27][32][32], zero for cout >= NOUT).
-__global__ void pack_kernel(const float *__restrict__ master, int NOUT,
-                            __bf16 *__restrict__ fwd, __bf16 *__restrict__ bwd) {
-  const int n = kTaps * 32 * 32;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const int tap = i / 1024, o = (i / 32) % 32, k = i % 32;
-    if (o < NOUT) fwd[((size_t)tap * NOUT + o) * kC + k] = f2bf(master[((size_t)tap * NOUT + o) * kC + k]);
-    const float vb = k < NOUT ? master[((size_t)(kTaps - 1 - tap) * NOUT + k) * kC + o] : 0.f;
-    bwd[((size_t)tap * 32 + o) * kC + k] = f2bf(vb);
-  }
-}
-
-// Input features of one sample (log10 n_H, log10 jH, FP32) -> BF16 channels
-// 0, 1 of the activation tensor (normalised), zeros elsewhere; an optional
-// crop [o..o+S) of a larger sample.
-__global__ void features_kernel(const float *__restrict__ feat, int D, int H, int W,
-                                int od, int oh, int ow, int S0, int S1, int S2,
-                                float m0, float s0, float m1, float s1,
-                                __bf16 *__restrict__ out) {
-  const size_t n = (size_t)S0 * S1 * S2;
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n * kC;
-       i += (size_t)gridDim.x * blockDim.x) {
-    const size_t v = i / kC;
-    const int c = (int)(i % kC);
-    float r = 0.f;
-    if (c < 2) {
-      const int z = (int)(v % S2), y = (int)((v / S2) % S1), xx = (int)(v / ((size_t)S1 * S2));
-      const size_t src = (((size_t)(od + xx) * H) + (oh + y)) * W + (ow + z);
-      r = c == 0 ? (feat[2 * src] - m0) * s0 : (feat[2 * src + 1] - m1) * s1;
+    const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    p[i] = pi;
+    int l = kLayers - 1;
+    while (i < L.off_w[l]) --l;
+    if (i < L.off_b[l]) {
+      const int j = (int)(i - L.off_w[l]), NOUT = L.nout[l];
+      const int k = j % kC, o = (j / kC) % NOUT, tap = j / (kC * NOUT);
+      L.fwd[l][j] = f2bf(pi);
+      L.bwd[l][((size_t)(kTaps - 1 - tap) * 32 + k) * kC + o] = f2bf(pi);
     }
-    out[i] = f2bf(r);
   }
 }
 
-__global__ void crop_target_kernel(const float *__restrict__ t, int D, int H, int W,
-                                   int od, int oh, int ow, int S0, int S1, int S2,
-                                   float inv_scale, float *__restrict__ out) {
+// Crops of the samples (features log10 n_H, log10 jH; FP32) as the network's
+// input, 2 normalised BF16 channels per voxel, and their scaled targets.
+constexpr int kMaxCrops = 16;
+struct Crops {
+  int sample[kMaxCrops], d[kMaxCrops], h[kMaxCrops], w[kMaxCrops];  // and origins
+};
+__device__ __forceinline__ uint32_t pack_features(float f0, float f1, float m0, float s0,
+                                                  float m1, float s1) {
+  union {
+    __bf16 c[2];
+    uint32_t u;
+  } o;
+  o.c[0] = f2bf((f0 - m0) * s0);
+  o.c[1] = f2bf((f1 - m1) * s1);
+  return o.u;
+}
+__global__ void crops_kernel(const float *__restrict__ feat, const float *__restrict__ tgt,
+                             int D, int H, int W, Crops C, int S0, int S1, int S2, float m0,
+                             float s0, float m1, float s1, float inv_scale,
+                             uint32_t *__restrict__ out, float *__restrict__ tgt_out) {
   const size_t n = (size_t)S0 * S1 * S2;
+  const int b = blockIdx.y;
+  const size_t base = (size_t)C.sample[b] * D * H * W;
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
        v += (size_t)gridDim.x * blockDim.x) {
     const int z = (int)(v % S2), y = (int)((v / S2) % S1), xx = (int)(v / ((size_t)S1 * S2));
-    out[v] = t[(((size_t)(od + xx) * H) + (oh + y)) * W + (ow + z)] * inv_scale;
+    const size_t src =
+        base + (((size_t)(C.d[b] + xx) * H) + (C.h[b] + y)) * W + (C.w[b] + z);
+    const float2 f = reinterpret_cast<const float2 *>(feat)[src];
+    out[b * n + v] = pack_features(f.x, f.y, m0, s0, m1, s1);
+    if (tgt) tgt_out[b * n + v] = tgt[src] * inv_scale;
   }
 }
 
@@ -476,7 +942,7 @@ __global__ void ctx_features_kernel(GridDev g, const double *__restrict__ n,
                                     const double *__restrict__ J,
                                     const double *__restrict__ xn, int mode, int D, int H,
                                     int W, double jconv, float m0, float s0, float m1,
-                                    float s1, __bf16 *__restrict__ act,
+                                    float s1, uint32_t *__restrict__ act,
                                     float *__restrict__ feat) {
   const size_t nv = (size_t)D * H * W;
   for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < nv;
@@ -490,16 +956,7 @@ __global__ void ctx_features_kernel(GridDev g, const double *__restrict__ n,
       feat[2 * v] = f0;
       feat[2 * v + 1] = f1;
     }
-    if (act) {
-      bf16x8 p0 = bf16x8{}, pz = bf16x8{};
-      p0[0] = f2bf((f0 - m0) * s0);
-      p0[1] = f2bf((f1 - m1) * s1);
-      bf16x8 *o = reinterpret_cast<bf16x8 *>(act + v * kC);
-      o[0] = p0;
-      o[1] = pz;
-      o[2] = pz;
-      o[3] = pz;
-    }
+    if (act) act[v] = pack_features(f0, f1, m0, s0, m1, s1);
   }
 }
 
@@ -601,12 +1058,6 @@ __global__ void zero_f32_kernel(float *p, size_t n) {
     p[i] = 0.f;
 }
 
-__global__ void zero_bf16_kernel(__bf16 *p, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (size_t)gridDim.x * blockDim.x)
-    p[i] = f2bf(0.f);
-}
-
 }  // namespace cmi
 
 using namespace cmi;
@@ -616,11 +1067,15 @@ using namespace cmi;
 // ---------------------------------------------------------------------------
 struct cmi_net {
   int device = 0;
+  int num_cus = 0;
   hipStream_t stream = nullptr;
   std::string err;
   size_t nparam = 0;
   size_t off_w[kLayers], off_b[kLayers];  // offsets into the master vector
-  float *p = nullptr, *g = nullptr, *m = nullptr, *v = nullptr;  // FP32
+  float *p = nullptr, *m = nullptr, *v = nullptr;  // FP32
+  float *g = nullptr;      // kCopies copies of the gradient and the loss
+  size_t grad_stride = 0;  // values from copy to copy
+  float *grad_sum = nullptr;  // their sum (loss_and_grad)
   __bf16 *wf[kLayers] = {}, *wb[kLayers] = {};                    // packed
   int step = 0;
   // normalisation of the features and of the target logits
@@ -633,15 +1088,17 @@ struct cmi_net {
   int dil[kLayers] = {1, 1, 1, 1};  // dilation of each layer's 3x3x3 taps
   float w_pos = 1.f;  // loss weight of predictions more neutral than the target
   int mode = 0;       // input mode of the warm start (0: jH, 1: refine x_n)
-  int tiled = 1;      // forward convolutions through conv3_tiled_kernel where it fits
+  int tiled = 1;      // forward convolutions through conv_block_kernel
   // dataset (device): features [S][N][2] FP32, targets [S][N] FP32
   float *ds_feat = nullptr, *ds_tgt = nullptr;
   int ds_n = 0, ds_dim[3] = {0, 0, 0};
   size_t ds_cap = 0;
   // work buffers (sized for the largest batch seen)
-  size_t work_vox = 0;
-  __bf16 *act[kLayers] = {};  // act[0] = input, act[l] = output of layer l-1
-  __bf16 *dact[2] = {};       // gradient ping-pong
+  size_t work_vox = 0, grad_vox = 0;
+  uint32_t *in = nullptr;     // the input, 2 BF16 channels per voxel
+  __bf16 *act[kLayers] = {};  // act[l] = output of layer l-1 (l >= 1)
+  __bf16 *dact[2] = {};       // gradient ping-pong (training only)
+  __bf16 *dz = nullptr;       // gradient of the output, one value per voxel
   float *z = nullptr, *tgt = nullptr, *loss = nullptr;
   float *feat_tmp = nullptr;
   size_t feat_cap = 0;
@@ -663,27 +1120,80 @@ int nfail(cmi_net *n, int code, const std::string &m) {
 
 int nout_of(int l) { return layer_cout(l) > 16 ? 32 : 16; }
 
-int ensure_work(cmi_net *n, size_t nvox) {
-  if (nvox <= n->work_vox) return CMI_OK;
-  for (int l = 0; l < kLayers; ++l) hipFree(n->act[l]);
-  for (int k = 0; k < 2; ++k) hipFree(n->dact[k]);
-  hipFree(n->z);
-  hipFree(n->tgt);
-  n->work_vox = 0;
-  for (int l = 0; l < kLayers; ++l) NET_TRY(n, hipMalloc(&n->act[l], nvox * kC * sizeof(__bf16)));
-  for (int k = 0; k < 2; ++k) NET_TRY(n, hipMalloc(&n->dact[k], nvox * kC * sizeof(__bf16)));
-  NET_TRY(n, hipMalloc(&n->z, nvox * sizeof(float)));
-  NET_TRY(n, hipMalloc(&n->tgt, nvox * sizeof(float)));
-  n->work_vox = nvox;
+// Work buffers for nvox voxels; the gradient's for training only.
+int ensure_work(cmi_net *n, size_t nvox, bool training) {
+  if (nvox > n->work_vox) {
+    n->work_vox = 0;
+    hipFree(n->in);
+    n->in = nullptr;
+    for (int l = 1; l < kLayers; ++l) {
+      hipFree(n->act[l]);
+      n->act[l] = nullptr;
+    }
+    hipFree(n->z);
+    hipFree(n->tgt);
+    n->z = n->tgt = nullptr;
+    NET_TRY(n, hipMalloc(&n->in, nvox * sizeof(uint32_t)));
+    for (int l = 1; l < kLayers; ++l)
+      NET_TRY(n, hipMalloc(&n->act[l], nvox * kC * sizeof(__bf16)));
+    NET_TRY(n, hipMalloc(&n->z, nvox * sizeof(float)));
+    NET_TRY(n, hipMalloc(&n->tgt, nvox * sizeof(float)));
+    n->work_vox = nvox;
+  }
+  if (training && nvox > n->grad_vox) {
+    n->grad_vox = 0;
+    for (int k = 0; k < 2; ++k) {
+      hipFree(n->dact[k]);
+      n->dact[k] = nullptr;
+    }
+    hipFree(n->dz);
+    n->dz = nullptr;
+    for (int k = 0; k < 2; ++k)
+      NET_TRY(n, hipMalloc(&n->dact[k], nvox * kC * sizeof(__bf16)));
+    NET_TRY(n, hipMalloc(&n->dz, nvox * sizeof(__bf16)));
+    n->grad_vox = nvox;
+  }
   return CMI_OK;
 }
 
+Layers layers_of(const cmi_net *n) {
+  Layers L;
+  for (int l = 0; l < kLayers; ++l) {
+    L.off_w[l] = n->off_w[l];
+    L.off_b[l] = n->off_b[l];
+    L.nout[l] = nout_of(l);
+    L.fwd[l] = n->wf[l];
+    L.bwd[l] = n->wb[l];
+  }
+  return L;
+}
+
 int pack(cmi_net *n) {
-  for (int l = 0; l < kLayers; ++l)
-    hipLaunchKernelGGL(pack_kernel, dim3(108), dim3(256), 0, n->stream, n->p + n->off_w[l],
-                       nout_of(l), n->wf[l], n->wb[l]);
+  hipLaunchKernelGGL(pack_kernel, dim3(27, kLayers), dim3(256), 0, n->stream, n->p,
+                     layers_of(n));
   NET_TRY(n, hipGetLastError());
   return CMI_OK;
+}
+
+// Blocks of bz x 8 x 8 voxels over B samples of D x H x W at a dilation.
+BlockGeo block_geo(int B, int D, int H, int W, int dil, int bz) {
+  BlockGeo G;
+  G.D = D;
+  G.H = H;
+  G.W = W;
+  G.dil = dil;
+  G.nrz = std::min(dil, D);
+  G.nry = std::min(dil, H);
+  G.nrx = std::min(dil, W);
+  auto blocks = [&](int extent, int edge) {
+    const int sub = (extent + dil - 1) / dil;
+    return (sub + edge - 1) / edge;
+  };
+  G.nbz = blocks(D, bz);
+  G.nby = blocks(H, kE);
+  G.nbx = blocks(W, kE);
+  G.nblocks = B * G.nrz * G.nry * G.nrx * G.nbz * G.nby * G.nbx;
+  return G;
 }
 
 unsigned grid_for(size_t items, unsigned per_block, unsigned cap = 65535) {
@@ -692,69 +1202,104 @@ unsigned grid_for(size_t items, unsigned per_block, unsigned cap = 65535) {
   return (unsigned)(g < cap ? g : cap);
 }
 
-// forward over act[0] (nvox voxels in B samples of D x H x W) -> z
+// The network's input from the features of B whole volumes.
+void input_features(cmi_net *n, const float *feat, int B, const int dim[3]) {
+  const size_t nv = (size_t)dim[0] * dim[1] * dim[2];
+  for (int b0 = 0; b0 < B; b0 += kMaxCrops) {
+    const int nb = std::min(kMaxCrops, B - b0);
+    Crops C{};
+    for (int b = 0; b < nb; ++b) C.sample[b] = b0 + b;
+    hipLaunchKernelGGL(crops_kernel, dim3(grid_for(nv, 256, 8192), nb), dim3(256), 0, n->stream,
+                       feat, (const float *)nullptr, dim[0], dim[1], dim[2], C, dim[0], dim[1],
+                       dim[2], n->mean[0], n->scale[0], n->mean[1], n->scale[1], 1.f,
+                       n->in + (size_t)b0 * nv, (float *)nullptr);
+  }
+}
+
+// forward over n->in (B samples of D x H x W) -> zout
 int forward(cmi_net *n, int B, int D, int H, int W, float *zout) {
   const int nrun = B * D * H * (W / 16);
-  const unsigned blocks = grid_for((size_t)nrun, 4, 1u << 30);  // one wave per run
+  const unsigned runs = grid_for((size_t)nrun, 4, 1u << 30);  // one wave per run
+  const __bf16 *const in = reinterpret_cast<const __bf16 *>(n->in);
   for (int l = 0; l < kLayers; ++l) {
     const float *bias = n->p + n->off_b[l];
     const int dil = n->dil[l];
-    if (n->tiled && tiled_shape_ok(D, H, W, dil)) {
-      // the same outputs, blocks of a dilation sub-lattice staged in LDS
-      const unsigned tb = (unsigned)((size_t)B * D * H * W / (16 * kTZ * kTY));
-      if (l < kLayers - 1)
-        hipLaunchKernelGGL(conv3_tiled_kernel<2>, dim3(tb), dim3(64 * kTiledWaves), 0,
-                           n->stream, n->act[l], n->wf[l], bias, D, H, W, dil, n->act[l + 1],
-                           (float *)nullptr, 1);
+    if (n->tiled) {
+      const BlockGeo G = block_geo(B, D, H, W, dil, kE);
+#define CMI_CONV(NB, FEAT, X, Y, YF, RELU)                                                \
+  hipLaunchKernelGGL((conv_block_kernel<NB, FEAT>), dim3(G.nblocks), dim3(kConvThreads), 0, \
+                     n->stream, G, X, n->wf[l], bias, Y, YF, (const __bf16 *)nullptr, RELU)
+      if (l == 0)
+        CMI_CONV(2, true, in, n->act[1], (float *)nullptr, 1);
+      else if (l < kLayers - 1)
+        CMI_CONV(2, false, n->act[l], n->act[l + 1], (float *)nullptr, 1);
       else
-        hipLaunchKernelGGL(conv3_tiled_kernel<1>, dim3(tb), dim3(64 * kTiledWaves), 0,
-                           n->stream, n->act[l], n->wf[l], bias, D, H, W, dil,
-                           (__bf16 *)nullptr, zout, 0);
+        CMI_CONV(1, false, n->act[l], (__bf16 *)nullptr, zout, 0);
+#undef CMI_CONV
       continue;
     }
-    if (l < kLayers - 1) {
-      hipLaunchKernelGGL(conv3_kernel<2>, dim3(blocks), dim3(256), 0, n->stream, n->act[l],
-                         n->wf[l], bias, nrun, D, H, W, n->dil[l], n->act[l + 1], (float *)nullptr,
-                         (const __bf16 *)nullptr, 1);
-    } else {
-      hipLaunchKernelGGL(conv3_kernel<1>, dim3(blocks), dim3(256), 0, n->stream, n->act[l],
-                         n->wf[l], bias, nrun, D, H, W, n->dil[l], (__bf16 *)nullptr, zout,
-                         (const __bf16 *)nullptr, 0);
-    }
+    if (l == 0)
+      hipLaunchKernelGGL((conv3_kernel<2, true>), dim3(runs), dim3(256), 0, n->stream, in,
+                         n->wf[l], bias, nrun, D, H, W, dil, n->act[1], (float *)nullptr, 1);
+    else if (l < kLayers - 1)
+      hipLaunchKernelGGL((conv3_kernel<2, false>), dim3(runs), dim3(256), 0, n->stream,
+                         n->act[l], n->wf[l], bias, nrun, D, H, W, dil, n->act[l + 1],
+                         (float *)nullptr, 1);
+    else
+      hipLaunchKernelGGL((conv3_kernel<1, false>), dim3(runs), dim3(256), 0, n->stream,
+                         n->act[l], n->wf[l], bias, nrun, D, H, W, dil, (__bf16 *)nullptr, zout,
+                         0);
   }
   NET_TRY(n, hipGetLastError());
   return CMI_OK;
 }
 
-// backward from the MSE loss on z vs tgt; gradients accumulate into n->g
+void zero_grad(cmi_net *n) {
+  hipLaunchKernelGGL(zero_f32_kernel, dim3(1024), dim3(256), 0, n->stream, n->g,
+                     kCopies * n->grad_stride);
+}
+
+// Workgroups of a weight gradient: two per CU, the blocks shared out evenly.
+unsigned grad_grid(const cmi_net *n, const BlockGeo &G) {
+  const int most = 2 * n->num_cus;
+  const int each = (G.nblocks + most - 1) / most;
+  return (unsigned)((G.nblocks + each - 1) / each);
+}
+
+// backward from the MSE loss on z vs tgt; the loss and the gradients add into
+// the copies in n->g
 int backward(cmi_net *n, int B, int D, int H, int W) {
+  static_assert(kLayers >= 3, "a first, a last and layers between");
   const size_t nvox = (size_t)B * D * H * W;
-  const int nrun = B * D * H * (W / 16);
-  const unsigned blocks = grid_for((size_t)nrun, 4, 1u << 30);  // one wave per run
-  const int nrow = B * D * H * (W / 32);
-  const int rows_per_wave = 16;
-  const int nchunks = (nrow + rows_per_wave - 1) / rows_per_wave;
+  const uint16_t *const dz = reinterpret_cast<const uint16_t *>(n->dz);
+  const int last = kLayers - 1;
+  hipLaunchKernelGGL(mse_kernel, dim3(grid_for(nvox, 1024, 512)), dim3(256), 0, n->stream,
+                     n->z, n->tgt, nvox, n->w_pos, n->dz, n->g, n->grad_stride, n->nparam,
+                     n->off_b[last]);
   __bf16 *dy = n->dact[0], *dx = n->dact[1];
-  hipLaunchKernelGGL(zero_bf16_kernel, dim3(grid_for(nvox * kC, 256, 4096)), dim3(256), 0,
-                     n->stream, dy, nvox * kC);
-  hipLaunchKernelGGL(mse_kernel, dim3(grid_for(nvox, 256, 1024)), dim3(256), 0, n->stream,
-                     n->z, n->tgt, nvox, n->w_pos, dy, n->loss);
-  for (int l = kLayers - 1; l >= 0; --l) {
-    const int NOUT = nout_of(l);
-    const int nb_out = NOUT / 16;
-    const size_t waves = (size_t)kTaps * nb_out * nchunks;
-    hipLaunchKernelGGL(wgrad_kernel, dim3(grid_for(waves, 4, 1u << 30)), dim3(256), 0, n->stream, dy,
-                       n->act[l], nb_out, nrow, rows_per_wave, D, H, W, n->dil[l],
-                       n->g + n->off_w[l], NOUT);
-    hipLaunchKernelGGL(bgrad_kernel, dim3(grid_for(nvox, 8, 2048)), dim3(256), 0, n->stream,
-                       dy, nvox, layer_cout(l), n->g + n->off_b[l]);
-    if (l > 0) {
-      // dx = conv(dy, flipped transposed W), masked by the ReLU of layer l-1
-      hipLaunchKernelGGL(conv3_kernel<2>, dim3(blocks), dim3(256), 0, n->stream, dy, n->wb[l],
-                         (const float *)nullptr, nrun, D, H, W, n->dil[l], dx, (float *)nullptr,
-                         (const __bf16 *)n->act[l], 0);
-      std::swap(dy, dx);
+  for (int l = last; l >= 0; --l) {
+    const BlockGeo Gw = block_geo(B, D, H, W, n->dil[l], kGZ);
+    const BlockGeo Gx = block_geo(B, D, H, W, n->dil[l], kE);
+    const unsigned wg = grad_grid(n, Gw);
+    if (l == last) {
+      hipLaunchKernelGGL(wgrad_last_kernel, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dz,
+                         n->act[l], n->g, n->grad_stride, n->off_w[l], nout_of(l));
+      hipLaunchKernelGGL(dgrad_last_kernel, dim3(Gx.nblocks), dim3(kConvThreads), 0, n->stream,
+                         Gx, dz, n->wb[l], n->act[l], dy);
+      continue;
     }
+    if (l == 0) {
+      hipLaunchKernelGGL(wgrad_first_kernel, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dy,
+                         n->in, n->g, n->grad_stride, n->off_w[l], n->off_b[l]);
+      continue;
+    }
+    hipLaunchKernelGGL(wgrad_block_kernel, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dy,
+                       n->act[l], n->g, n->grad_stride, n->off_w[l], n->off_b[l]);
+    // dx = conv(dy, flipped transposed W), masked by the ReLU of layer l-1
+    hipLaunchKernelGGL((conv_block_kernel<2, false>), dim3(Gx.nblocks), dim3(kConvThreads), 0,
+                       n->stream, Gx, dy, n->wb[l], (const float *)nullptr, dx, (float *)nullptr,
+                       n->act[l], 0);
+    std::swap(dy, dx);
   }
   NET_TRY(n, hipGetLastError());
   return CMI_OK;
@@ -771,6 +1316,11 @@ int cmi_net_create(uint64_t seed, cmi_net **out) {
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return CMI_ERR_NODEVICE;
   cmi_net *n = new cmi_net();
   (void)hipGetDevice(&n->device);
+  if (hipDeviceGetAttribute(&n->num_cus, hipDeviceAttributeMultiprocessorCount, n->device) !=
+      hipSuccess) {
+    delete n;
+    return CMI_ERR_HIP;
+  }
   size_t off = 0;
   for (int l = 0; l < kLayers; ++l) {
     n->off_w[l] = off;
@@ -781,7 +1331,9 @@ int cmi_net_create(uint64_t seed, cmi_net **out) {
   n->nparam = off;
   hipError_t e = hipStreamCreateWithFlags(&n->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc(&n->p, off * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&n->g, off * sizeof(float));
+  n->grad_stride = (off + 1 + 63) / 64 * 64;
+  if (e == hipSuccess) e = hipMalloc(&n->g, kCopies * n->grad_stride * sizeof(float));
+  if (e == hipSuccess) e = hipMalloc(&n->grad_sum, n->grad_stride * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&n->m, off * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&n->v, off * sizeof(float));
   if (e == hipSuccess) e = hipMalloc(&n->loss, 65536 * sizeof(float));
@@ -827,6 +1379,7 @@ void cmi_net_destroy(cmi_net *n) {
   if (n->stream) (void)hipStreamSynchronize(n->stream);
   hipFree(n->p);
   hipFree(n->g);
+  hipFree(n->grad_sum);
   hipFree(n->m);
   hipFree(n->v);
   hipFree(n->loss);
@@ -835,7 +1388,9 @@ void cmi_net_destroy(cmi_net *n) {
     hipFree(n->wb[l]);
     hipFree(n->act[l]);
   }
+  hipFree(n->in);
   for (int k = 0; k < 2; ++k) hipFree(n->dact[k]);
+  hipFree(n->dz);
   hipFree(n->z);
   hipFree(n->tgt);
   hipFree(n->ds_feat);
@@ -978,43 +1533,38 @@ int cmi_net_train(cmi_net *n, int steps, int batch, const int crop[3], float lr,
   if (crop[2] % 32 != 0) return nfail(n, CMI_ERR_ARG, "crop: last extent must be a multiple of 32");
   (void)hipSetDevice(n->device);
   const size_t cv = (size_t)crop[0] * crop[1] * crop[2];
-  int rc = ensure_work(n, cv * batch);
+  int rc = ensure_work(n, cv * batch, true);
   if (rc != CMI_OK) return rc;
-  const size_t nv = (size_t)n->ds_dim[0] * n->ds_dim[1] * n->ds_dim[2];
-  hipLaunchKernelGGL(zero_f32_kernel, dim3(64), dim3(256), 0, n->stream, n->loss, (size_t)steps);
   const float b1 = 0.9f, b2 = 0.999f;
   for (int s = 0; s < steps; ++s) {
-    for (int b = 0; b < batch; ++b) {
-      const u32x4 r = philox4x32_10(u32x4{(uint32_t)s, (uint32_t)b, (uint32_t)n->step, 0x7A1Eu},
-                                    (uint32_t)seed, (uint32_t)(seed >> 32));
-      const int si = (int)(r.x % (uint32_t)n->ds_n);
-      const int od = (int)(r.y % (uint32_t)(n->ds_dim[0] - crop[0] + 1));
-      const int oh = (int)(r.z % (uint32_t)(n->ds_dim[1] - crop[1] + 1));
-      const int ow = (int)(r.w % (uint32_t)(n->ds_dim[2] - crop[2] + 1));
-      hipLaunchKernelGGL(features_kernel, dim3(grid_for(cv * kC, 256, 4096)), dim3(256), 0,
-                         n->stream, n->ds_feat + (size_t)si * nv * 2, n->ds_dim[0],
-                         n->ds_dim[1], n->ds_dim[2], od, oh, ow, crop[0], crop[1], crop[2],
-                         n->mean[0], n->scale[0], n->mean[1], n->scale[1],
-                         n->act[0] + (size_t)b * cv * kC);
-      hipLaunchKernelGGL(crop_target_kernel, dim3(grid_for(cv, 256, 4096)), dim3(256), 0,
-                         n->stream, n->ds_tgt + (size_t)si * nv, n->ds_dim[0], n->ds_dim[1],
-                         n->ds_dim[2], od, oh, ow, crop[0], crop[1], crop[2],
-                         1.f / n->out_scale, n->tgt + (size_t)b * cv);
+    for (int b0 = 0; b0 < batch; b0 += kMaxCrops) {
+      const int nb = std::min(kMaxCrops, batch - b0);
+      Crops C{};
+      for (int b = 0; b < nb; ++b) {
+        const u32x4 r =
+            philox4x32_10(u32x4{(uint32_t)s, (uint32_t)(b0 + b), (uint32_t)n->step, 0x7A1Eu},
+                          (uint32_t)seed, (uint32_t)(seed >> 32));
+        C.sample[b] = (int)(r.x % (uint32_t)n->ds_n);
+        C.d[b] = (int)(r.y % (uint32_t)(n->ds_dim[0] - crop[0] + 1));
+        C.h[b] = (int)(r.z % (uint32_t)(n->ds_dim[1] - crop[1] + 1));
+        C.w[b] = (int)(r.w % (uint32_t)(n->ds_dim[2] - crop[2] + 1));
+      }
+      hipLaunchKernelGGL(crops_kernel, dim3(grid_for(cv, 256, 4096), nb), dim3(256), 0,
+                         n->stream, n->ds_feat, n->ds_tgt, n->ds_dim[0], n->ds_dim[1],
+                         n->ds_dim[2], C, crop[0], crop[1], crop[2], n->mean[0], n->scale[0],
+                         n->mean[1], n->scale[1], 1.f / n->out_scale, n->in + (size_t)b0 * cv,
+                         n->tgt + (size_t)b0 * cv);
     }
-    hipLaunchKernelGGL(zero_f32_kernel, dim3(64), dim3(256), 0, n->stream, n->g, n->nparam);
+    zero_grad(n);
     rc = forward(n, batch, crop[0], crop[1], crop[2], n->z);
     if (rc != CMI_OK) return rc;
-    float *loss_slot = n->loss + s;
-    std::swap(n->loss, loss_slot);  // backward accumulates into n->loss
     rc = backward(n, batch, crop[0], crop[1], crop[2]);
-    std::swap(n->loss, loss_slot);
     if (rc != CMI_OK) return rc;
     ++n->step;
     const float c1 = 1.f - powf(b1, (float)n->step), c2 = 1.f - powf(b2, (float)n->step);
-    hipLaunchKernelGGL(adam_kernel, dim3(128), dim3(256), 0, n->stream, n->p, n->g, n->m, n->v,
-                       n->nparam, lr, b1, b2, 1e-8f, c1, c2, 0.f);
-    rc = pack(n);
-    if (rc != CMI_OK) return rc;
+    hipLaunchKernelGGL(adam_kernel, dim3(grid_for(n->nparam, 256, 1024)), dim3(256), 0,
+                       n->stream, n->p, n->g, n->grad_stride, n->m, n->v, n->nparam, lr, b1, b2,
+                       1e-8f, c1, c2, 0.f, layers_of(n), n->loss + s);
   }
   NET_TRY(n, hipGetLastError());
   if (losses)
@@ -1034,7 +1584,7 @@ int cmi_net_loss_and_grad(cmi_net *n, const float *feat, const float *target, in
   (void)hipSetDevice(n->device);
   NET_TRY(n, hipStreamSynchronize(n->stream));  // null-stream copies below
   const size_t nv = (size_t)dim[0] * dim[1] * dim[2];
-  int rc = ensure_work(n, nv * B);
+  int rc = ensure_work(n, nv * B, true);
   if (rc != CMI_OK) return rc;
   std::vector<float> ts(target, target + nv * B);
   for (float &t : ts) t /= n->out_scale;
@@ -1047,18 +1597,18 @@ int cmi_net_loss_and_grad(cmi_net *n, const float *feat, const float *target, in
     hipFree(df);
     return nfail(n, CMI_ERR_HIP, "loss_and_grad: copy failed");
   }
-  for (int b = 0; b < B; ++b)
-    hipLaunchKernelGGL(features_kernel, dim3(grid_for(nv * kC, 256, 4096)), dim3(256), 0,
-                       n->stream, df + (size_t)b * nv * 2, dim[0], dim[1], dim[2], 0, 0, 0,
-                       dim[0], dim[1], dim[2], n->mean[0], n->scale[0], n->mean[1],
-                       n->scale[1], n->act[0] + (size_t)b * nv * kC);
-  hipLaunchKernelGGL(zero_f32_kernel, dim3(64), dim3(256), 0, n->stream, n->g, n->nparam);
-  hipLaunchKernelGGL(zero_f32_kernel, dim3(1), dim3(64), 0, n->stream, n->loss, (size_t)1);
+  input_features(n, df, B, dim);
+  zero_grad(n);
   rc = forward(n, B, dim[0], dim[1], dim[2], n->z);
   if (rc == CMI_OK) rc = backward(n, B, dim[0], dim[1], dim[2]);
   if (rc == CMI_OK) {
-    e = hipMemcpyAsync(grad, n->g, n->nparam * sizeof(float), hipMemcpyDeviceToHost, n->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(loss, n->loss, sizeof(float), hipMemcpyDeviceToHost, n->stream);
+    hipLaunchKernelGGL(sum_grad_kernel, dim3(grid_for(n->nparam, 256, 1024)), dim3(256), 0,
+                       n->stream, n->g, n->grad_stride, n->nparam, n->grad_sum);
+    e = hipMemcpyAsync(grad, n->grad_sum, n->nparam * sizeof(float), hipMemcpyDeviceToHost,
+                       n->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(loss, n->grad_sum + n->nparam, sizeof(float), hipMemcpyDeviceToHost,
+                         n->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(n->stream);
     if (e != hipSuccess) rc = nfail(n, CMI_ERR_HIP, "loss_and_grad failed");
   }
@@ -1073,7 +1623,7 @@ int cmi_net_predict(cmi_net *n, const float *feat, const int dim[3], float *logi
   (void)hipSetDevice(n->device);
   NET_TRY(n, hipStreamSynchronize(n->stream));  // null-stream copies below
   const size_t nv = (size_t)dim[0] * dim[1] * dim[2];
-  int rc = ensure_work(n, nv);
+  int rc = ensure_work(n, nv, false);
   if (rc != CMI_OK) return rc;
   if (n->feat_cap < nv) {
     hipFree(n->feat_tmp);
@@ -1083,9 +1633,7 @@ int cmi_net_predict(cmi_net *n, const float *feat, const int dim[3], float *logi
     n->feat_cap = nv;
   }
   NET_TRY(n, hipMemcpy(n->feat_tmp, feat, nv * 2 * sizeof(float), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(features_kernel, dim3(grid_for(nv * kC, 256, 8192)), dim3(256), 0,
-                     n->stream, n->feat_tmp, dim[0], dim[1], dim[2], 0, 0, 0, dim[0], dim[1],
-                     dim[2], n->mean[0], n->scale[0], n->mean[1], n->scale[1], n->act[0]);
+  input_features(n, n->feat_tmp, 1, dim);
   rc = forward(n, 1, dim[0], dim[1], dim[2], n->z);
   if (rc != CMI_OK) return rc;
   NET_TRY(n, hipMemcpyAsync(logits, n->z, nv * sizeof(float), hipMemcpyDeviceToHost, n->stream));
@@ -1122,14 +1670,14 @@ int cmi_net_warm_start(cmi_net *n, cmi_ctx *c, double luminosity, uint64_t npack
   if (W % 16 != 0) return nfail(n, CMI_ERR_ARG, "ncell[2] must be a multiple of 16");
   (void)hipSetDevice(n->device);
   const size_t nv = (size_t)D * H * W;
-  rc = ensure_work(n, nv);
+  rc = ensure_work(n, nv, false);
   if (rc != CMI_OK) return rc;
   NET_TRY(n, hipStreamSynchronize(c->stream));  // the first pass has finished
   hipLaunchKernelGGL(ctx_features_kernel, dim3(grid_for(nv, 256, 8192)), dim3(256), 0,
                      n->stream, c->g, (const double *)c->f.n, (const double *)c->f.J,
                      (const double *)c->f.xn, n->mode, D, H, W,
                      context_jconv(c, luminosity, npackets), n->mean[0], n->scale[0],
-                     n->mean[1], n->scale[1], n->act[0], (float *)nullptr);
+                     n->mean[1], n->scale[1], n->in, (float *)nullptr);
   rc = forward(n, 1, D, H, W, n->z);
   if (rc != CMI_OK) return rc;
   const bool fp32 = c->precision == CMI_PREC_FP32;
@@ -1214,7 +1762,7 @@ int cmi_net_context_features(cmi_net *n, cmi_ctx *c, double luminosity, uint64_t
                      n->stream, c->g, (const double *)c->f.n, (const double *)c->f.J,
                      (const double *)c->f.xn, n->mode, D, H, W,
                      context_jconv(c, luminosity, npackets), 0.f, 1.f, 0.f, 1.f,
-                     (__bf16 *)nullptr, d);
+                     (uint32_t *)nullptr, d);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess)
     e = hipMemcpyAsync(features, d, nv * 2 * sizeof(float), hipMemcpyDeviceToHost, n->stream);
