@@ -39,36 +39,21 @@ int ilog2_exact(int v) {
   return ((1 << s) == v) ? s : -1;
 }
 
-// Device cell index of (subgrid, ix, iy, iz): mirrors cell_addr().
-inline size_t dev_index(const cmi_ctx *c, size_t sub, int ix, int iy, int iz) {
-  const GridDev &g = c->g;
-  const int tx = ix >> g.tshift[0], ty = iy >> g.tshift[1],
-            tz = iz >> g.tshift[2];
-  const int lx = ix - (tx << g.tshift[0]), ly = iy - (ty << g.tshift[1]),
-            lz = iz - (tz << g.tshift[2]);
-  const size_t t = ((size_t)tx * g.ntile[1] + ty) * g.ntile[2] + tz;
-  const size_t l = ((((size_t)lx << g.tshift[1]) + ly) << g.tshift[2]) + lz;
-  return sub * (size_t)g.cps + t * (size_t)g.tile_cells + l;
+// Fields between the caller's order and the device's, those of the two whose
+// host array is given.
+hipError_t put_fields(cmi_ctx *c, CellField a, CellField b = {}) {
+  CellField f[2];
+  int nf = 0;
+  if (a.host) f[nf++] = a;
+  if (b.host) f[nf++] = b;
+  return c->stage.upload_cells(c->device, c->stream, cell_order(c->g), c->ncell_total, f, nf);
 }
-
-// Reference order (subgrid-major, ix*ny*nz+iy*nz+iz) <-> device order.
-template <class T>
-void to_device_order(const cmi_ctx *c, const T *ref, std::vector<T> &dev) {
-  dev.resize(c->ncell_total);
-  size_t r = 0;
-  for (size_t s = 0; s < c->nsubgrid; ++s)
-    for (int ix = 0; ix < c->sc[0]; ++ix)
-      for (int iy = 0; iy < c->sc[1]; ++iy)
-        for (int iz = 0; iz < c->sc[2]; ++iz) dev[dev_index(c, s, ix, iy, iz)] = ref[r++];
-}
-
-template <class T>
-void from_device_order(const cmi_ctx *c, const std::vector<T> &dev, T *ref) {
-  size_t r = 0;
-  for (size_t s = 0; s < c->nsubgrid; ++s)
-    for (int ix = 0; ix < c->sc[0]; ++ix)
-      for (int iy = 0; iy < c->sc[1]; ++iy)
-        for (int iz = 0; iz < c->sc[2]; ++iz) ref[r++] = dev[dev_index(c, s, ix, iy, iz)];
+hipError_t get_fields(cmi_ctx *c, CellField a, CellField b = {}) {
+  CellField f[2];
+  int nf = 0;
+  if (a.host) f[nf++] = a;
+  if (b.host) f[nf++] = b;
+  return c->stage.download_cells(c->device, c->stream, cell_order(c->g), c->ncell_total, f, nf);
 }
 
 // Largest power of two <= cap that divides v.
@@ -203,11 +188,7 @@ ReemitDraws list_reemit_draws(const cmi_ctx *c) {
 // n_H of a context in the reference layout (for the result writers)
 int get_density_ref(cmi_ctx *c, double *nH) {
   (void)hipSetDevice(c->device);
-  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
-  std::vector<double> d(c->ncell_total);
-  CMI_TRY_HIP(c, hipMemcpy(d.data(), c->f.n, d.size() * sizeof(double),
-                           hipMemcpyDeviceToHost));
-  from_device_order(c, d, nH);
+  CMI_TRY_HIP(c, get_fields(c, CellField{nH, c->f.n, 1.}));
   return CMI_OK;
 }
 }  // namespace cmi
@@ -338,9 +319,11 @@ int cmi_create(const double box[6], const int ncell[3], const int nsub[3],
     return CMI_ERR_HIP;
   }
   // DensitySubGrid.hpp:544-551: n = 1e8, x_n = 1e-6, J = 0
-  std::vector<double> n0(c->ncell_total, 1.e8), x0(c->ncell_total, 1.e-6);
-  int rc = cmi_set_fields(c, n0.data(), x0.data());
-  if (rc == CMI_OK) rc = cmi_reset_intensity(c);
+  e = launch_fill(c->f.n, c->ncell_total, 1.e8, c->stream);
+  if (e == hipSuccess) e = launch_fill(c->f.xn, c->ncell_total, 1.e-6, c->stream);
+  if (e == hipSuccess && precision == CMI_PREC_FP32)
+    e = launch_kappa(c->f, c->ncell_total, c->sigma * delta0(c), c->stream);
+  int rc = e == hipSuccess ? cmi_reset_intensity(c) : CMI_ERR_HIP;
   // the allocation-free entry point's scratch address on this device
   if (rc == CMI_OK) rc = noalloc_setup(c);
   if (rc != CMI_OK) {
@@ -387,10 +370,7 @@ int cmi_set_engine(cmi_ctx *c, int engine, const cmi_tuning *t) {
         std::vector<double> n(c->ncell_total), x(c->ncell_total), J(c->ncell_total);
         int rc = cmi_get_fields(c, J.data(), x.data());
         if (rc != CMI_OK) return rc;
-        std::vector<double> nd(c->ncell_total);
-        CMI_TRY_HIP(c, hipMemcpy(nd.data(), c->f.n, c->ncell_total * sizeof(double),
-                                 hipMemcpyDeviceToHost));
-        from_device_order(c, nd, n.data());
+        CMI_TRY_HIP(c, get_fields(c, CellField{n.data(), c->f.n, 1.}));
         const int old_tile[3] = {c->tile[0], c->tile[1], c->tile[2]};
         rc = set_tile(c, tile);
         if (rc != CMI_OK) {
@@ -411,63 +391,34 @@ int cmi_set_engine(cmi_ctx *c, int engine, const cmi_tuning *t) {
 int cmi_set_fields(cmi_ctx *c, const double *nH, const double *xn) {
   if (!c) return CMI_ERR_ARG;
   (void)hipSetDevice(c->device);
-  // the copies below go through the null stream, which does not wait for
-  // the context's non-blocking stream: work still queued there (a
-  // restriction or prolongation, a warm start) must not land after them
-  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
-  std::vector<double> d;
-  if (nH) {
-    to_device_order(c, nH, d);
-    CMI_TRY_HIP(c, hipMemcpy(c->f.n, d.data(), d.size() * sizeof(double),
-                             hipMemcpyHostToDevice));
-  }
-  if (xn) {
-    to_device_order(c, xn, d);
-    CMI_TRY_HIP(c, hipMemcpy(c->f.xn, d.data(), d.size() * sizeof(double),
-                             hipMemcpyHostToDevice));
-  }
+  // on the context's stream, behind what is queued there (a restriction or
+  // prolongation, a warm start)
+  CMI_TRY_HIP(c, put_fields(c, CellField{const_cast<double *>(nH), c->f.n, 1.},
+                            CellField{const_cast<double *>(xn), c->f.xn, 1.}));
   if (c->precision == CMI_PREC_FP32) {
     CMI_TRY_HIP(c, launch_kappa(c->f, c->ncell_total, c->sigma * delta0(c),
                                 c->stream));
-    CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
   }
+  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
   return CMI_OK;
 }
 
 int cmi_set_intensity(cmi_ctx *c, const double *J) {
   if (!c || !J) return CMI_ERR_ARG;
   (void)hipSetDevice(c->device);
-  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));  // as in cmi_set_fields
-  std::vector<double> d;
-  to_device_order(c, J, d);
-  if (c->precision == CMI_PREC_FP32) {
-    const double inv = 1. / (c->sigma * delta0(c));
-    for (double &v : d) v *= inv;
-  }
-  CMI_TRY_HIP(c, hipMemcpy(c->f.J, d.data(), d.size() * sizeof(double),
-                           hipMemcpyHostToDevice));
+  const double scale = c->precision == CMI_PREC_FP32 ? 1. / (c->sigma * delta0(c)) : 1.;
+  CMI_TRY_HIP(c, put_fields(c, CellField{const_cast<double *>(J), c->f.J, scale}));
+  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
   return CMI_OK;
 }
 
 int cmi_get_fields(cmi_ctx *c, double *J, double *xn) {
   if (!c) return CMI_ERR_ARG;
   (void)hipSetDevice(c->device);
-  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
-  std::vector<double> d(c->ncell_total);
-  if (J) {
-    CMI_TRY_HIP(c, hipMemcpy(d.data(), c->f.J, d.size() * sizeof(double),
-                             hipMemcpyDeviceToHost));
-    if (c->precision == CMI_PREC_FP32) {
-      const double s = c->sigma * delta0(c);
-      for (double &v : d) v *= s;
-    }
-    from_device_order(c, d, J);
-  }
-  if (xn) {
-    CMI_TRY_HIP(c, hipMemcpy(d.data(), c->f.xn, d.size() * sizeof(double),
-                             hipMemcpyDeviceToHost));
-    from_device_order(c, d, xn);
-  }
+  const double scale = c->precision == CMI_PREC_FP32 ? c->sigma * delta0(c) : 1.;
+  CMI_TRY_HIP(c, get_fields(c, CellField{J, c->f.J, scale}, CellField{xn, c->f.xn, 1.}));
+  // with neither array: what is queued has been done
+  if (!J && !xn) CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
   return CMI_OK;
 }
 

@@ -8,6 +8,7 @@
 
 #include "../../include/cmi.h"
 #include "cmi_internal.hpp"
+#include "cmi_stage.hpp"
 
 namespace cmi {
 struct TilesEngine;
@@ -45,6 +46,7 @@ struct cmi_ctx {
   uint64_t kernel_calls = 0;
   int kernel_timing = 1;  // record the tiles engine's per-round process events
   cmi::TilesEngine *tiles = nullptr;
+  cmi::Stage stage;  // host <-> device transfers
   std::string err;
 };
 
