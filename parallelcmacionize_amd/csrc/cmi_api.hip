@@ -295,8 +295,8 @@ int cmi_create(const double box[6], const int ncell[3], const int nsub[3],
   if (e == hipSuccess) e = hipMalloc(&c->f.J, c->ncell_total * sizeof(double));
   if (e == hipSuccess && precision == CMI_PREC_FP32)
     e = hipMalloc(&c->f.kappa, c->ncell_total * sizeof(float));
-  if (e == hipSuccess) e = hipMalloc(&c->d_cnt, sizeof(Counters));
-  if (e == hipSuccess) e = hipHostMalloc(&c->h_cnt, sizeof(Counters));
+  if (e == hipSuccess) e = hipMalloc(&c->d_cnt, kCounterCopies * sizeof(Counters));
+  if (e == hipSuccess) e = hipHostMalloc(&c->h_cnt, kCounterCopies * sizeof(Counters));
   if (e == hipSuccess) e = hipMalloc(&c->d_src, sizeof(SourcesDev));
   if (e == hipSuccess) e = hipHostMalloc(&c->h_src, sizeof(SourcesDev));
   if (e == hipSuccess) e = hipMalloc(&c->d_partial, kIonizeBlocks * sizeof(double));
@@ -519,7 +519,7 @@ int cmi_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub,
                                           hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(ds, start_sub, n * sizeof(uint32_t),
                                           hipMemcpyHostToDevice, c->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(c->d_cnt, 0, sizeof(Counters), c->stream);
+  if (e == hipSuccess) e = clear_counters(c);
   if (e == hipSuccess) e = hipEventRecord(c->ev0, c->stream);
   if (e == hipSuccess)
     e = launch_walk_list(c->g, c->f, c->precision, dp, ds, n, dst, dc, dh,
@@ -533,9 +533,7 @@ int cmi_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub,
     e = hipMemcpyAsync(crossings, dc, n * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream);
   if (e == hipSuccess && hops)
     e = hipMemcpyAsync(hops, dh, n * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(Counters),
-                                          hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = fetch_counters(c, c->d_cnt);
   float ms = 0.f;
   if (e == hipSuccess) e = hipEventElapsedTime(&ms, c->ev0, c->ev1);
   hipFree(dp);
@@ -632,15 +630,13 @@ int cmi_transport(cmi_ctx *c, uint64_t npackets, uint64_t seed,
   re.iteration = iteration;
   const int blocks = c->tuning.walk_blocks > 0 ? c->tuning.walk_blocks
                                                : c->num_cus * 8;
-  CMI_TRY_HIP(c, hipMemsetAsync(c->d_cnt, 0, sizeof(Counters), c->stream));
+  CMI_TRY_HIP(c, clear_counters(c));
   CMI_TRY_HIP(c, hipEventRecord(c->ev0, c->stream));
   CMI_TRY_HIP(c, launch_walk_emit(c->g, c->f, c->precision, c->d_src, npackets,
                                   iteration, seed, sigma, blocks, re, c->d_cnt,
                                   c->stream));
   CMI_TRY_HIP(c, hipEventRecord(c->ev1, c->stream));
-  CMI_TRY_HIP(c, hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(Counters),
-                                hipMemcpyDeviceToHost, c->stream));
-  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
+  CMI_TRY_HIP(c, fetch_counters(c, c->d_cnt));
   float ms = 0.f;
   CMI_TRY_HIP(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
   c->kernel_time_sum += ms * 1e-3;

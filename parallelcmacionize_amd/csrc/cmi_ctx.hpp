@@ -106,6 +106,20 @@ inline void source_counts(const std::vector<double> &L, uint64_t npackets,
   for (uint64_t r = 0; r < rem; ++r) counts[order[r % (uint64_t)nsrc]]++;
 }
 
+// The transport counters cleared (a fill kernel) and, once the stream has
+// finished, read back into h_cnt[0].
+inline hipError_t clear_counters(cmi_ctx *c) {
+  return launch_fill(reinterpret_cast<double *>(c->d_cnt),
+                     kCounterCopies * sizeof(Counters) / sizeof(double), 0., c->stream);
+}
+inline hipError_t fetch_counters(cmi_ctx *c, const Counters *from) {
+  hipError_t e = hipMemcpyAsync(c->h_cnt, from, kCounterCopies * sizeof(Counters),
+                                hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) sum_counters(c->h_cnt);
+  return e;
+}
+
 // Shared by the explicit-list transports (cmi_api.hip).
 int prepare_list_transport(cmi_ctx *c, const cmi_photon *p,
                            const uint32_t *start_sub, size_t n);

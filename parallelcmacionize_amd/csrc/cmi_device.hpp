@@ -165,8 +165,14 @@ __device__ __forceinline__ int emit_packet(const SourcesDev &S, uint64_t k,
   return s;
 }
 
-// Counters a transport writes back (device-side, one slot each).
-struct Counters {
+// Counters a transport writes back.  A context keeps kCounterCopies of them, a
+// cache line or two each: a workgroup adds its sums to the copy of its index,
+// and the host adds the copies up.  Atomic adds to one line pass one at a time
+// (about 10 ns each for the whole chip): with one add per wave and counter on
+// one copy, a transport of 3e6 packets through 120x96x72 cells took 2.5 ms,
+// with these copies 1.1; 1e8 packets through 256^3 cells 30.4 and 26.8.
+constexpr int kCounterCopies = 64;
+struct alignas(128) Counters {
   unsigned long long crossings;
   unsigned long long hops;
   unsigned long long absorbed;
@@ -177,6 +183,55 @@ struct Counters {
   unsigned long long walkout_crossings;  // of crossings: those of walk-out launches
   unsigned long long walkout_hops;       // of hops: tile legs of walk-out launches
 };
+
+// The copies summed into the first.
+inline void sum_counters(Counters *c) {
+  for (int i = 1; i < kCounterCopies; ++i) {
+    c->crossings += c[i].crossings;
+    c->hops += c[i].hops;
+    c->absorbed += c[i].absorbed;
+    c->escaped += c[i].escaped;
+    c->errors += c[i].errors;
+    c->reemitted += c[i].reemitted;
+    c->walkout_crossings += c[i].walkout_crossings;
+    c->walkout_hops += c[i].walkout_hops;
+  }
+}
+
+// What one lane counted.
+struct LaneCounts {
+  unsigned long long crossings, hops, absorbed, escaped, errors, reemitted,
+      walkout_crossings, walkout_hops;
+};
+
+// A workgroup's counts to its copy: summed within the waves, then through LDS
+// (sh: one row per wave), then one atomic per counter.  Every thread of the
+// workgroup calls it.
+constexpr int kCountFields = 8;
+__device__ __forceinline__ void add_counts(Counters *__restrict__ cnt, const LaneCounts &v,
+                                           unsigned long long (*sh)[kCountFields]) {
+  const unsigned long long f[kCountFields] = {v.crossings, v.hops,      v.absorbed,
+                                              v.escaped,   v.errors,    v.reemitted,
+                                              v.walkout_crossings, v.walkout_hops};
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < kCountFields; ++k) {
+    unsigned long long s = f[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) sh[wave][k] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x < kCountFields) {
+    unsigned long long s = 0;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) s += sh[w][threadIdx.x];
+    Counters &c = cnt[blockIdx.x % kCounterCopies];
+    unsigned long long *const to[kCountFields] = {
+        &c.crossings, &c.hops,      &c.absorbed,          &c.escaped,
+        &c.errors,    &c.reemitted, &c.walkout_crossings, &c.walkout_hops};
+    if (s) atomicAdd(to[threadIdx.x], s);
+  }
+}
 
 // ---------------------------------------------------------------------------
 // Reemission draws (do_reemission, testDensitySubGrid_omp.cpp:675-702: a

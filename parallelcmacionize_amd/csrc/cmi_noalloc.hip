@@ -31,7 +31,7 @@ constexpr size_t kOffStatus = align256(kOffSub + kMaxPackets * sizeof(uint32_t))
 constexpr size_t kOffCross = align256(kOffStatus + kMaxPackets * sizeof(int32_t));
 constexpr size_t kOffHops = align256(kOffCross + kMaxPackets * sizeof(uint32_t));
 constexpr size_t kOffCnt = align256(kOffHops + kMaxPackets * sizeof(uint32_t));
-constexpr size_t kScratchBytes = align256(kOffCnt + sizeof(Counters));
+constexpr size_t kScratchBytes = align256(kOffCnt + cmi::kCounterCopies * sizeof(Counters));
 static_assert(sizeof(Counters) % sizeof(double) == 0,
               "the counters are cleared as doubles");
 
@@ -105,7 +105,8 @@ int cmi_transport_packets_noalloc(cmi_ctx *c, cmi_photon *p,
   // the previous call's counters are still there: clear them with a fill
   // kernel (no memset node, should a caller capture the stream)
   CMI_TRY_HIP(c, launch_fill(reinterpret_cast<double *>(cnt),
-                             sizeof(Counters) / sizeof(double), 0., c->stream));
+                             kCounterCopies * sizeof(Counters) / sizeof(double), 0.,
+                             c->stream));
   CMI_TRY_HIP(c, hipEventRecord(c->ev0, c->stream));
   CMI_TRY_HIP(c, launch_walk_list(c->g, c->f, c->precision, dp, ds, n, dst, dc,
                                   dh, list_reemit_draws(c), cnt, c->stream));
@@ -121,9 +122,7 @@ int cmi_transport_packets_noalloc(cmi_ctx *c, cmi_photon *p,
   if (hops)
     CMI_TRY_HIP(c, hipMemcpyAsync(hops, dh, n * sizeof(uint32_t),
                                   hipMemcpyDeviceToHost, c->stream));
-  CMI_TRY_HIP(c, hipMemcpyAsync(c->h_cnt, cnt, sizeof(Counters),
-                                hipMemcpyDeviceToHost, c->stream));
-  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
+  CMI_TRY_HIP(c, fetch_counters(c, cnt));
   float ms = 0.f;
   CMI_TRY_HIP(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
   fill_ctx_stats(c, stats, n, ms * 1e-3);

@@ -826,6 +826,8 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
     return reinterpret_cast<Acc *>(accB + o * (uint32_t)(sizeof(Acc) / sizeof(float)));
   };
   __shared__ uint32_t s_next, s_surv, s_desc;
+  __shared__ unsigned long long s_cross;
+  __shared__ unsigned long long s_counts[kThreads / 64][kCountFields];
   __shared__ uint32_t s_face[6];
   __shared__ uint32_t s_fbase[6];
   __shared__ uint32_t s_nbr[6];  // the tile's face neighbours, by exit face
@@ -833,6 +835,7 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
   const int lane = threadIdx.x & 63;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const uint32_t ndesc = *ndesc_ptr;
+  if (blockIdx.x >= ndesc) return;  // no visit for this workgroup
   const int T0 = kTile ? kTile : G.T[0], T1 = kTile ? kTile : G.T[1],
             T2 = kTile ? kTile : G.T[2];
   const int st0 = (T1 * T2) << 2, st1 = T2 << 2;  // byte strides
@@ -843,11 +846,13 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
 
   // a workgroup's first visit is the descriptor of its own index; later ones
   // come from the ticket, counted on from the grid size (no start-of-launch
-  // queue of every workgroup on the one counter)
+  // queue of every workgroup on the one counter, and none at the end of a
+  // round that has no more visits than workgroups)
   bool first = true;
   for (;;) {
     uint32_t di = blockIdx.x;
     if (!first) {
+      if (ndesc <= gridDim.x) break;
       if (threadIdx.x == 0) s_desc = gridDim.x + atomicAdd(ticket, 1u);
       __syncthreads();
       di = s_desc;
@@ -870,6 +875,7 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
       if (threadIdx.x == 0) {
         s_next = kThreads;  // the first kThreads packets are claimed below
         s_surv = 0;
+        s_cross = 0;
       }
       if (threadIdx.x < 6) s_face[threadIdx.x] = 0;
     }
@@ -1155,6 +1161,13 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
         const Acc v = accL[i];
         if (v != (Acc)0) atomicAdd(&Jt[i], AccAtomic<Acc>::value(v, G.fix_inv));
       }
+      if (prob_cross) {
+        // crossings of this visit, per problem (one atomic per visit)
+        unsigned long long v = my_cross - cross0;  // this visit, widened
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        if (lane == 0) atomicAdd(&s_cross, v);
+      }
       const uint32_t ns = s_surv;
       for (uint32_t i = ns + threadIdx.x; i < D.count; i += kThreads)
         dest_out[D.start + i] = kNone;
@@ -1188,40 +1201,12 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
           if (i < ns) rel_out[D.start + i] = s_fbase[v[k] >> 29] + (v[k] & ((1u << 29) - 1u));
         }
       }
-      if (prob_cross) {
-        // crossings of this visit, per problem (one atomic per wave)
-        unsigned long long v = my_cross - cross0;  // this visit, widened
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if (lane == 0 && v) atomicAdd(&prob_cross[prob], v);
-      }
+      if (prob_cross && threadIdx.x == 0 && s_cross)
+        atomicAdd(&prob_cross[prob], s_cross);
     }
     __syncthreads();
   }
-  // kernel-wide counters
-  unsigned long long w_cross = my_cross, w_hops = my_hops, w_abs = my_abs, w_esc = my_esc,
-                     w_err = my_err;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    w_cross += __shfl_xor(w_cross, o, 64);
-    w_hops += __shfl_xor(w_hops, o, 64);
-    w_abs += __shfl_xor(w_abs, o, 64);
-    w_esc += __shfl_xor(w_esc, o, 64);
-    w_err += __shfl_xor(w_err, o, 64);
-  }
-  if (lane == 0) {
-    if (w_cross) atomicAdd(&cnt->crossings, w_cross);
-    if (w_hops) atomicAdd(&cnt->hops, w_hops);
-    if (w_abs) atomicAdd(&cnt->absorbed, w_abs);
-    if (w_esc) atomicAdd(&cnt->escaped, w_esc);
-    if (w_err) atomicAdd(&cnt->errors, w_err);
-  }
-  if (kReemit) {
-    unsigned long long w_re = my_re;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) w_re += __shfl_xor(w_re, o, 64);
-    if (lane == 0 && w_re) atomicAdd(&cnt->reemitted, w_re);
-  }
+  add_counts(cnt, LaneCounts{my_cross, my_hops, my_abs, my_esc, my_err, my_re, 0, 0}, s_counts);
 }
 
 // A deposit of the walk-out: the value a visit's accumulator adds for it.
@@ -1356,36 +1341,15 @@ __global__ void __launch_bounds__(kThreads) tiles_walkout_kernel(
       po.final_tile[pid] = tile;
     }
   }
-  unsigned long long w_cross = my_cross, w_hops = my_hops, w_abs = my_abs, w_esc = my_esc,
-                     w_err = my_err;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    w_cross += __shfl_xor(w_cross, o, 64);
-    w_hops += __shfl_xor(w_hops, o, 64);
-    w_abs += __shfl_xor(w_abs, o, 64);
-    w_esc += __shfl_xor(w_esc, o, 64);
-    w_err += __shfl_xor(w_err, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    if (w_cross) atomicAdd(&cnt->crossings, w_cross);
-    if (w_hops) atomicAdd(&cnt->hops, w_hops);
-    if (w_abs) atomicAdd(&cnt->absorbed, w_abs);
-    if (w_esc) atomicAdd(&cnt->escaped, w_esc);
-    if (w_err) atomicAdd(&cnt->errors, w_err);
-    if (w_cross) atomicAdd(&cnt->walkout_crossings, w_cross);
-    if (w_hops) atomicAdd(&cnt->walkout_hops, w_hops);
-  }
+  __shared__ unsigned long long s_counts[kThreads / 64][kCountFields];
+  add_counts(cnt, LaneCounts{my_cross, my_hops, my_abs, my_esc, my_err, 0, my_cross, my_hops},
+             s_counts);
 }
 
 __global__ void zero_u32_kernel(uint32_t *p, size_t n) {
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (size_t)gridDim.x * blockDim.x)
     p[i] = 0;
-}
-
-__global__ void zero_counters_kernel(Counters *c) {
-  if (threadIdx.x < sizeof(Counters) / 8)
-    reinterpret_cast<unsigned long long *>(c)[threadIdx.x] = 0;
 }
 
 // Final FP32 records of an explicit-list transport -> absolute positions.
@@ -1931,7 +1895,7 @@ int tiles_transport(cmi_ctx *c, uint64_t npackets, uint64_t seed,
   const RoundCfg R = round_cfg(c, G, (size_t)npackets);
   if (R.lds > kLdsBytes)
     return fail(c, CMI_ERR_ARG, "tiles engine: the tile's opacity and accumulator exceed the LDS");
-  hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, c->stream, c->d_cnt);
+  CMI_TRY_HIP(c, clear_counters(c));
   CMI_TRY_HIP(c, hipEventRecord(c->ev0, c->stream));
   // round 0: per-tile counts from the source split, planned, then the
   // emission fills the records and the index list
@@ -1947,9 +1911,7 @@ int tiles_transport(cmi_ctx *c, uint64_t npackets, uint64_t seed,
   rc = run_rounds(c, G, R, false, po, (size_t)npackets, &rounds);
   if (rc != CMI_OK) return rc;
   CMI_TRY_HIP(c, hipEventRecord(c->ev1, c->stream));
-  CMI_TRY_HIP(c, hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(Counters),
-                                hipMemcpyDeviceToHost, c->stream));
-  CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
+  CMI_TRY_HIP(c, fetch_counters(c, c->d_cnt));
   float ms = 0.f;
   CMI_TRY_HIP(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
   fill_stats_tiles(c, stats, npackets, rounds, ms * 1e-3);
@@ -2003,8 +1965,8 @@ int tiles_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub
     cleanup();
     return fail(c, CMI_ERR_HIP, "tiles list transport: copy failed");
   }
-  hipLaunchKernelGGL(zero_counters_kernel, dim3(1), dim3(64), 0, c->stream, c->d_cnt);
-  err = hipEventRecord(c->ev0, c->stream);
+  err = clear_counters(c);
+  if (err == hipSuccess) err = hipEventRecord(c->ev0, c->stream);
   if (err != hipSuccess) {
     cleanup();
     return fail(c, CMI_ERR_HIP, "tiles list transport: event record failed");
@@ -2038,9 +2000,7 @@ int tiles_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub
     err = hipMemcpyAsync(crossings, dc, n * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream);
   if (err == hipSuccess && hops)
     err = hipMemcpyAsync(hops, dh, n * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream);
-  if (err == hipSuccess)
-    err = hipMemcpyAsync(c->h_cnt, c->d_cnt, sizeof(Counters), hipMemcpyDeviceToHost, c->stream);
-  if (err == hipSuccess) err = hipStreamSynchronize(c->stream);
+  if (err == hipSuccess) err = fetch_counters(c, c->d_cnt);
   float ms = 0.f;
   if (err == hipSuccess) err = hipEventElapsedTime(&ms, c->ev0, c->ev1);
   cleanup();

@@ -337,14 +337,6 @@ __device__ __forceinline__ int visit_open(const Walker<T> &w, const GridDev &g) 
   return inside3(w.idx, g.sc) ? kContinue : kLeft;
 }
 
-// Wave-level sum of a 64-bit counter; lane 0 adds it to *dst.
-__device__ __forceinline__ void wave_add(unsigned long long *dst,
-                                         unsigned long long v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  if ((threadIdx.x & 63) == 0 && v) atomicAdd(dst, v);
-}
-
 // ---------------------------------------------------------------------------
 // Kernel: DensitySubGrid::interact on one subgrid for an explicit packet list
 // (the deterministic oracle's entry point).  One thread per packet.
@@ -479,12 +471,8 @@ __global__ void walk_list_kernel(GridDev g, Mode m, PhotonRec *p,
     my_err = (st < 0);
     my_re = nre;
   }
-  wave_add(&cnt->crossings, my_cross);
-  wave_add(&cnt->hops, my_hops);
-  wave_add(&cnt->absorbed, my_abs);
-  wave_add(&cnt->escaped, my_esc);
-  wave_add(&cnt->errors, my_err);
-  wave_add(&cnt->reemitted, my_re);
+  __shared__ unsigned long long sh[4][kCountFields];
+  add_counts(cnt, LaneCounts{my_cross, my_hops, my_abs, my_esc, my_err, my_re, 0, 0}, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -617,12 +605,8 @@ __global__ void __launch_bounds__(256, 4) walk_emit_kernel(
   __syncthreads();
   for (int i = threadIdx.x; i < (int)kHotCrossings * kHotPart; i += blockDim.x)
     if (hot.key[i] != kHotFree) atomicAdd(&m.J[hot.key[i]], hot.val[i]);
-  wave_add(&cnt->crossings, my_cross);
-  wave_add(&cnt->hops, my_hops);
-  wave_add(&cnt->absorbed, my_abs);
-  wave_add(&cnt->escaped, my_esc);
-  wave_add(&cnt->errors, my_err);
-  wave_add(&cnt->reemitted, my_re);
+  __shared__ unsigned long long sh[4][kCountFields];
+  add_counts(cnt, LaneCounts{my_cross, my_hops, my_abs, my_esc, my_err, my_re, 0, 0}, sh);
 }
 
 // ---------------------------------------------------------------------------
