@@ -1663,14 +1663,6 @@ struct RoundCfg {
   unsigned place_blocks;
 };
 
-// A round with fewer packets than (resident workgroups / kMinVisitsDiv) full
-// chunks is cut into about that many visits.  Measured on the 256^3 clumpy
-// workload (1e8 packets, 768 resident workgroups): cutting the last ~15
-// rounds, whose largest visits then set the round's time, saves 2 % of the
-// transport; cutting earlier rounds (4 or 1 visits per workgroup) costs more
-// in per-visit latency (descriptor, opacity staging, flush) than it gains.
-constexpr uint32_t kMinVisitsDiv = 4;
-
 static RoundCfg round_cfg(const cmi_ctx *c, const TileGeo &G, size_t n0) {
   RoundCfg r;
   r.threads = c->tuning.block_threads == 256 ? 256 : 512;
@@ -1681,9 +1673,17 @@ static RoundCfg round_cfg(const cmi_ctx *c, const TileGeo &G, size_t n0) {
   r.fp32acc = c->tuning.lds_fp32 != 0;
   r.lds = ((sizeof(float) * (size_t)(G.W.pad + G.tile_cells) + 15) & ~(size_t)15) +
           (size_t)G.tile_cells * (r.fp32acc ? sizeof(float) : sizeof(double));
-  const int wg_per_cu = (int)std::max<size_t>(1, std::min<size_t>(8, (160 * 1024) / (r.lds + 1024)));
+  // resident workgroups: by LDS, and by registers (6 waves per SIMD)
+  const size_t by_lds = (160 * 1024) / (r.lds + 1024), by_waves = 24 / (size_t)(r.threads / 64);
+  const int wg_per_cu = (int)std::max<size_t>(1, std::min(by_lds, by_waves));
   r.grid = c->num_cus * wg_per_cu;
-  r.min_visits = std::max<uint32_t>(1, (uint32_t)r.grid / kMinVisitsDiv);
+  // A round with fewer packets than full chunks for every resident workgroup
+  // is cut into about one visit for each (chunks of kChunkFloor at least): the
+  // largest visits set such a round's time.  A quarter, a half, one visit per
+  // workgroup, transport only: 64^3, 1e6 packets, 10 iterations 4.30, 3.84,
+  // 3.77 ms; reemission 128^3, 5e6, 3 iterations 14.8, 13.7, 13.2; 256^3, 1e7,
+  // 5 iterations 20.2, 19.5, 18.9; 256^3, 1e8, 10 iterations 268, 265, 263.
+  r.min_visits = (uint32_t)r.grid;
   // walk-out: when a check of the packets left (at the start and every
   // kRoundsPerCheck rounds) finds at most finish_max, one launch walks them
   // all to the end.  Default: one packet per resident lane.  Measured on the
