@@ -17,11 +17,11 @@
 //             (LDS-counter compaction) with their destination tile; the
 //             per-face exit counts go to the next round's tile histogram
 //             (whose old values are the visit's bases) and every survivor
-//             gets its position relative to its destination's segment;
+//             keeps its exit face and its rank among the visit's exits there;
 //   plan      one workgroup: exclusive scan of the histogram into tile
 //             segments, and the next round's work descriptors (tile, start,
 //             count) in chunks, smaller ones for rounds with few packets;
-//   place     segment start + relative position of every survivor -> the
+//   place     segment start + visit's base + rank of every survivor -> the
 //             index list the next round gathers packets through.
 //
 // Round 0 has no visits before it: for emitted packets its per-tile counts
@@ -176,6 +176,14 @@ struct Desc {
   uint32_t start;
   uint32_t count;
   uint32_t pad;
+};
+
+// What a visit leaves for the placement of its survivors (slots start ..
+// start + ns - 1): every exit face's neighbour tile (kNone without exits) and
+// the visit's base within that tile's next segment.
+struct alignas(64) VisitOut {
+  uint32_t start, ns;
+  uint32_t nbr[6], base[6];
 };
 
 // Per-packet outputs of explicit-list transports (indexed by packet id).
@@ -425,7 +433,8 @@ static const uint32_t kChunk = 8192;      // packets per workgroup visit
 static const uint32_t kChunkFloor = 256;  // smallest chunk accepted
 
 // total[0]: packets of the round being planned (in: those of the round just
-// processed, kept in total[1] for the placement); nonempty (optional) counts
+// processed, kept in total[1]); ndesc[0]: its visits (those of the round just
+// processed are kept in ndesc[1] for the placement); nonempty (optional) counts
 // the plans that found packets.  A round's chunk is `chunk`, or smaller when
 // the round holds fewer than min_visits * chunk packets: then the chunk is cut
 // (down to kChunkFloor) so that the round still has about min_visits visits.
@@ -450,6 +459,7 @@ __global__ void __launch_bounds__(kPlanThreads) tiles_plan_kernel(
   const bool track = prob_round != nullptr;
   if (threadIdx.x == 0) {
     total[1] = total[0];
+    ndesc[1] = ndesc[0];
     s_ncrowded = 0;
   }
   if (track)
@@ -661,20 +671,50 @@ __global__ void __launch_bounds__(kScatterThreads) tiles_scatter_kernel(
 }
 
 // Placement of one round's survivors: the process kernel left each survivor
-// slot its position relative to its destination tile's segment (the visit's
-// base for that face, reserved by the histogram atomic, plus the survivor's
-// rank among the visit's exits through that face), so the index list is one
-// streaming pass without atomics.
-__global__ void tiles_place_kernel(const uint32_t *__restrict__ nslots_ptr,
-                                   const uint32_t *__restrict__ dest,
-                                   const uint32_t *__restrict__ rel,
-                                   const uint32_t *__restrict__ seg,
-                                   uint32_t *__restrict__ idx) {
-  const uint32_t n = *nslots_ptr;
-  for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < n;
-       s += gridDim.x * blockDim.x) {
-    const uint32_t t = dest[s];
-    if (t != kNone) idx[seg[t] + rel[s]] = s;
+// slot its exit face and its rank among its visit's exits through that face,
+// and the visit's neighbour and base per face (reserved by the histogram
+// atomic).  With the segments of the next round planned, the index list is one
+// streaming pass without atomics, 4 B read and 4 B written per survivor, a
+// piece of kPlacePiece slots of a visit to a workgroup.  With a destination
+// tile and a finished position per slot instead, written and rewritten by the
+// process kernel and read here, 256^3, 1e8 packets took 26.4 ms a transport;
+// with the visits' tables 24.7.
+constexpr int kPlaceThreads = 256;
+constexpr uint32_t kPlacePiece = 4096;
+constexpr uint32_t kRankMask = (1u << 29) - 1u;
+
+__global__ void __launch_bounds__(kPlaceThreads) tiles_place_kernel(
+    const uint32_t *__restrict__ nvisits_ptr, uint32_t pieces_per_visit,
+    const VisitOut *__restrict__ visits, const uint32_t *__restrict__ rel,
+    const uint32_t *__restrict__ seg, uint32_t *__restrict__ idx) {
+  __shared__ uint32_t s_at[6];
+  const uint32_t items = *nvisits_ptr * pieces_per_visit;
+  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
+    const uint32_t v = item / pieces_per_visit;
+    const uint32_t i0 = (item - v * pieces_per_visit) * kPlacePiece;
+    const uint32_t ns = visits[v].ns, start = visits[v].start;
+    if (i0 >= ns) continue;
+    __syncthreads();
+    if (threadIdx.x < 6) {
+      const uint32_t t = visits[v].nbr[threadIdx.x];
+      s_at[threadIdx.x] = t == kNone ? 0u : seg[t] + visits[v].base[threadIdx.x];
+    }
+    __syncthreads();
+    const uint32_t i1 = min(ns, i0 + kPlacePiece);
+    constexpr int kAhead = 8;
+    for (uint32_t i = i0 + threadIdx.x; i < i1; i += kAhead * kPlaceThreads) {
+      uint32_t r[kAhead];
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const uint32_t j = i + (uint32_t)k * kPlaceThreads;
+        r[k] = j < i1 ? rel[start + j] : 0u;
+      }
+#pragma unroll
+      for (int k = 0; k < kAhead; ++k) {
+        const uint32_t j = i + (uint32_t)k * kPlaceThreads;
+        if (j < i1) idx[s_at[r[k] >> 29] + (r[k] & kRankMask)] = start + j;
+      }
+    }
   }
 }
 
@@ -782,12 +822,12 @@ __device__ __forceinline__ void dda_axis(int l, float p, float d, float &tm,
 // iteration, with the absorption point's coordinate bits, the tile and the
 // packet's reemission count as the counter.
 template <class Acc, int kThreads, bool kList, bool kReemit = false, int kTile = 0>
-__global__ void __launch_bounds__(kThreads) tiles_process_kernel(
+__global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
     TileGeo G, const float *__restrict__ kappa, double *__restrict__ J,
     const Desc *__restrict__ desc, const uint32_t *__restrict__ ndesc_ptr,
     unsigned *__restrict__ ticket, const Rec32 *__restrict__ Pin,
     const uint32_t *__restrict__ idx, Rec32 *__restrict__ Pout,
-    uint32_t *__restrict__ dest_out, uint32_t *__restrict__ hist_next,
+    VisitOut *__restrict__ visit_out, uint32_t *__restrict__ hist_next,
     const uint32_t *__restrict__ pid_in, uint32_t *__restrict__ pid_out,
     PacketOut po, Counters *__restrict__ cnt,
     unsigned long long *__restrict__ prob_cross, int refill_batch,
@@ -798,6 +838,9 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
   // kTile > 0: the kernel serves kTile^3 tiles only, from a static block
   // whose address the compiler folds into the LDS instructions' offsets;
   // kTile = 0: any shape, dynamic LDS.
+  // Six waves per SIMD (80 VGPRs), the three workgroups per CU that the LDS
+  // of 16^3 tiles holds: at 82 VGPRs (five waves, two workgroups) 256^3, 1e8
+  // packets takes 8 % longer.
   constexpr int kCellsF = kTile * kTile * kTile;
   constexpr WalkLayout kWF = walk_layout(kTile ? kTile : 1, kTile ? kTile : 1, kTile ? kTile : 1);
   constexpr size_t kStatBytes =
@@ -829,8 +872,6 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
   __shared__ unsigned long long s_cross;
   __shared__ unsigned long long s_counts[kThreads / 64][kCountFields];
   __shared__ uint32_t s_face[6];
-  __shared__ uint32_t s_fbase[6];
-  __shared__ uint32_t s_nbr[6];  // the tile's face neighbours, by exit face
 
   const int lane = threadIdx.x & 63;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
@@ -891,12 +932,6 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
     const int nb_zp = tile_index(P, ttx, tty, ttz + 1), nb_zn = tile_index(P, ttx, tty, ttz - 1);
     const int ox = ttx << G.tshift[0], oy = tty << G.tshift[1],
               oz = ttz << G.tshift[2];
-    // exit face f = 2 axis + (negative direction): its neighbour tile
-    if (threadIdx.x < 6) {
-      const int f = threadIdx.x;
-      s_nbr[f] = (uint32_t)(f == 0 ? nb_xp : f == 1 ? nb_xn : f == 2 ? nb_yp
-                            : f == 3 ? nb_yn : f == 4 ? nb_zp : nb_zn);
-    }
 
     // prefetched next record of this lane
     bool has_nxt = false;
@@ -982,11 +1017,11 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
           const uint32_t slot = D.start + sbase + (uint32_t)__popcll(mv & lt);
           Pout[slot] = r;
           const float de = exit_axis == 0 ? d0 : (exit_axis == 1 ? d1 : d2);
+          // exit face f = 2 axis + (negative direction)
           const uint32_t f = 2u * (uint32_t)exit_axis + (de > 0.f ? 0u : 1u);
-          dest_out[slot] = s_nbr[f];
           if (kList) pid_out[slot] = my_pid;
           // the rank among this visit's exits through this face; the
-          // face's base is added once the visit has ended
+          // placement adds the face's base
           rel_out[slot] = (f << 29) | atomicAdd(&s_face[f], 1u);
         } else if (kList) {
           po.final_a[my_pid] = make_float4(q0, q1, q2, d0);
@@ -1154,7 +1189,7 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
       }
     }
     __syncthreads();
-    // flush the visit: J deposits, tail of the output region, face counts
+    // flush the visit: J deposits, face counts
     {
       double *Jt = J + (size_t)tile * tile_cells;
       for (int i = threadIdx.x; i < tile_cells; i += kThreads) {
@@ -1168,39 +1203,21 @@ __global__ void __launch_bounds__(kThreads) tiles_process_kernel(
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
         if (lane == 0) atomicAdd(&s_cross, v);
       }
-      const uint32_t ns = s_surv;
-      for (uint32_t i = ns + threadIdx.x; i < D.count; i += kThreads)
-        dest_out[D.start + i] = kNone;
       if (threadIdx.x < 6) {
         // the next round's count of each neighbour; the old value is this
         // visit's base within the neighbour's segment
-        const uint32_t c = s_face[threadIdx.x];
-        uint32_t base = 0;
-        if (c) {
-          const int f = threadIdx.x;
-          const int nt = f == 0 ? nb_xp : f == 1 ? nb_xn : f == 2 ? nb_yp
+        const int f = threadIdx.x;
+        const uint32_t c = s_face[f];
+        const int nt = f == 0 ? nb_xp : f == 1 ? nb_xn : f == 2 ? nb_yp
                        : f == 3 ? nb_yn : f == 4 ? nb_zp : nb_zn;
-          base = atomicAdd(&hist_next[nt], c);
-        }
-        s_fbase[threadIdx.x] = base;
+        visit_out[di].nbr[f] = c ? (uint32_t)nt : kNone;
+        visit_out[di].base[f] = c ? atomicAdd(&hist_next[nt], c) : 0u;
+      }
+      if (threadIdx.x == 0) {
+        visit_out[di].start = D.start;
+        visit_out[di].ns = s_surv;
       }
       __syncthreads();
-      // eight loads in flight per thread, then their rewrites: a loop of
-      // one load, wait and store per slot pays a memory latency per slot
-      constexpr int kFix = 8;
-      for (uint32_t i0 = threadIdx.x; i0 < ns; i0 += kFix * kThreads) {
-        uint32_t v[kFix];
-#pragma unroll
-        for (int k = 0; k < kFix; ++k) {
-          const uint32_t i = i0 + (uint32_t)k * kThreads;
-          v[k] = i < ns ? rel_out[D.start + i] : 0u;
-        }
-#pragma unroll
-        for (int k = 0; k < kFix; ++k) {
-          const uint32_t i = i0 + (uint32_t)k * kThreads;
-          if (i < ns) rel_out[D.start + i] = s_fbase[v[k] >> 29] + (v[k] & ((1u << 29) - 1u));
-        }
-      }
       if (prob_cross && threadIdx.x == 0 && s_cross)
         atomicAdd(&prob_cross[prob], s_cross);
     }
@@ -1433,7 +1450,8 @@ struct TilesEngine {
   int nprob = 0;
   size_t desc_cap = 0;
   Rec32 *P[2] = {nullptr, nullptr};
-  uint32_t *dest[2] = {nullptr, nullptr};
+  uint32_t *dest = nullptr;     // tiles of an explicit list's packets (round 0)
+  VisitOut *visits = nullptr;
   uint32_t *pid[2] = {nullptr, nullptr};
   uint32_t *idx = nullptr;
   uint32_t *rel = nullptr;      // survivors' positions in their next segment
@@ -1470,9 +1488,10 @@ static void free_engine(TilesEngine *e) {
   if (e->graph) hipGraphDestroy(e->graph);
   for (int i = 0; i < 2; ++i) {
     hipFree(e->P[i]);
-    hipFree(e->dest[i]);
     hipFree(e->pid[i]);
   }
+  hipFree(e->dest);
+  hipFree(e->visits);
   hipFree(e->idx);
   hipFree(e->rel);
   hipFree(e->hist);
@@ -1595,16 +1614,17 @@ static int ensure_engine(cmi_ctx *c, const std::vector<ProbGeo> &probs,
   hipError_t err = hipSuccess;
   for (int i = 0; i < 2 && err == hipSuccess; ++i) {
     err = hipMalloc(&e->P[i], cap * sizeof(Rec32));
-    if (err == hipSuccess) err = hipMalloc(&e->dest[i], cap * sizeof(uint32_t));
     if (err == hipSuccess && with_pid) err = hipMalloc(&e->pid[i], cap * sizeof(uint32_t));
   }
+  if (err == hipSuccess && with_pid) err = hipMalloc(&e->dest, cap * sizeof(uint32_t));
+  if (err == hipSuccess) err = hipMalloc(&e->visits, e->desc_cap * sizeof(VisitOut));
   if (err == hipSuccess) err = hipMalloc(&e->idx, cap * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->rel, cap * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->hist, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->seg, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->cursor, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->desc, e->desc_cap * sizeof(Desc));
-  if (err == hipSuccess) err = hipMalloc(&e->ndesc, sizeof(uint32_t));
+  if (err == hipSuccess) err = hipMalloc(&e->ndesc, 2 * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->total, 3 * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->ticket, sizeof(unsigned));
   if (err == hipSuccess) err = hipHostMalloc(&e->h_total, 3 * sizeof(uint32_t));
@@ -1699,7 +1719,7 @@ static RoundCfg round_cfg(const cmi_ctx *c, const TileGeo &G, size_t n0) {
                                : (uint32_t)((size_t)r.grid * r.threads));
   const size_t per_block = (size_t)kScatterThreads * kScatterItems;
   r.scatter_blocks = (unsigned)std::min<size_t>(8192, (n0 + per_block - 1) / per_block + 1);
-  r.place_blocks = (unsigned)std::min<size_t>(8192, (n0 + 4 * 256 - 1) / (4 * 256) + 1);
+  r.place_blocks = (unsigned)std::min<size_t>(8 * c->num_cus, n0 / 1024 + 1);
   return r;
 }
 
@@ -1710,7 +1730,7 @@ static void launch_process(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
 #define CMI_PROC(ACC, TH, LIST, RE, TL)                                            \
   hipLaunchKernelGGL((tiles_process_kernel<ACC, TH, LIST, RE, TL>), dim3(R.grid), dim3(TH), \
                      (TL) ? 0 : R.lds, c->stream, G, c->f.kappa, c->f.J, e->desc,      \
-                     e->ndesc, e->ticket, e->P[0], e->idx, e->P[1], e->dest[1], e->hist, \
+                     e->ndesc, e->ticket, e->P[0], e->idx, e->P[1], e->visits, e->hist, \
                      LIST ? e->pid[0] : nullptr, LIST ? e->pid[1] : nullptr, po,       \
                      c->d_cnt, prob_cross, R.refill, e->rel)
   // 16^3 tiles at 512 threads (the tuned shape): the kernel specialised to
@@ -1773,6 +1793,14 @@ static void launch_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
                      e->d_round_ctr, nonempty ? e->total + 2 : nullptr);
 }
 
+// The placement of a planned round's packets: the survivors of the one before.
+static void launch_place(cmi_ctx *c, const RoundCfg &R) {
+  TilesEngine *e = c->tiles;
+  hipLaunchKernelGGL(tiles_place_kernel, dim3(R.place_blocks), dim3(kPlaceThreads), 0,
+                     c->stream, e->ndesc + 1, (R.chunk + kPlacePiece - 1) / kPlacePiece,
+                     e->visits, e->rel, e->seg, e->idx);
+}
+
 // The host checks the packets left every kRoundsPerCheck rounds: a check
 // costs a host round trip (about 30 us), a round launched after the last
 // packet has gone about 20 us (its kernels find no work).
@@ -1801,18 +1829,15 @@ static int run_rounds(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool with
   while (r < max_rounds && !drained) {
     const int r_end = std::min(max_rounds, r + kRoundsPerCheck);
     for (; r < r_end; ++r) {
-      // round r reads P[0] (through idx) and writes its survivors to P[1];
-      // the plan keeps the round's count in total[1] for the placement
+      // round r reads P[0] (through idx) and writes its survivors to P[1]
       if (r < timed) CMI_TRY_HIP(c, hipEventRecord(e->ev[2 * r], c->stream));
       launch_process(c, G, R, with_pid, po, nullptr);
       if (r < timed) CMI_TRY_HIP(c, hipEventRecord(e->ev[2 * r + 1], c->stream));
       CMI_TRY_HIP(c, hipGetLastError());
       launch_plan(c, G, R, false, true);
-      hipLaunchKernelGGL(tiles_place_kernel, dim3(R.place_blocks), dim3(256), 0, c->stream,
-                         e->total + 1, e->dest[1], e->rel, e->seg, e->idx);
+      launch_place(c, R);
       CMI_TRY_HIP(c, hipGetLastError());
       std::swap(e->P[0], e->P[1]);
-      std::swap(e->dest[0], e->dest[1]);
       if (with_pid) std::swap(e->pid[0], e->pid[1]);
     }
     CMI_TRY_HIP(c, hipMemcpyAsync(e->h_total, e->total, 3 * sizeof(uint32_t),
@@ -1972,7 +1997,7 @@ int tiles_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub
     return fail(c, CMI_ERR_HIP, "tiles list transport: event record failed");
   }
   hipLaunchKernelGGL(tiles_load_list_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256),
-                     0, c->stream, G, c->g, dp, ds, n, e->P[0], e->dest[0], e->pid[0],
+                     0, c->stream, G, c->g, dp, ds, n, e->P[0], e->dest, e->pid[0],
                      e->hist);
   const RoundCfg R = round_cfg(c, G, n);
   if (R.lds > kLdsBytes) {
@@ -1982,7 +2007,7 @@ int tiles_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub
   // round 0: planned from the loaded histogram, index list by destination
   launch_plan(c, G, R, false);
   hipLaunchKernelGGL(tiles_scatter_kernel, dim3(R.scatter_blocks), dim3(kScatterThreads),
-                     0, c->stream, e->total, e->dest[0], e->seg, e->cursor, e->idx);
+                     0, c->stream, e->total, e->dest, e->seg, e->cursor, e->idx);
   PacketOut po{dst, dc, dh, fa, fb, dtile};
   uint32_t rounds = 0;
   rc = run_rounds(c, G, R, true, po, n, &rounds);
