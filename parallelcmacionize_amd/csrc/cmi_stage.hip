@@ -164,31 +164,4 @@ hipError_t Stage::download_cells(int device, hipStream_t st, const CellOrder &o,
              });
 }
 
-hipError_t Stage::upload(int device, hipStream_t st, const void *host, void *dev,
-                         size_t bytes) {
-  return run(device, bytes, 1,
-             [&](int s, int, size_t off, size_t len, bool begin) -> hipError_t {
-               if (!begin) return hipSuccess;
-               memcpy(h_[s], static_cast<const unsigned char *>(host) + off, len);
-               const hipError_t e = hipMemcpyAsync(static_cast<unsigned char *>(dev) + off, h_[s],
-                                                   len, hipMemcpyHostToDevice, st);
-               return e == hipSuccess ? hipEventRecord(ev_[s], st) : e;
-             });
-}
-
-hipError_t Stage::download(int device, hipStream_t st, const void *dev, void *host,
-                           size_t bytes) {
-  return run(device, bytes, 1,
-             [&](int s, int, size_t off, size_t len, bool begin) -> hipError_t {
-               if (!begin) {
-                 memcpy(static_cast<unsigned char *>(host) + off, h_[s], len);
-                 return hipSuccess;
-               }
-               const hipError_t e = hipMemcpyAsync(
-                   h_[s], static_cast<const unsigned char *>(dev) + off, len,
-                   hipMemcpyDeviceToHost, st);
-               return e == hipSuccess ? hipEventRecord(ev_[s], st) : e;
-             });
-}
-
 }  // namespace cmi

@@ -1,6 +1,5 @@
-// cmi_stage.hpp -- host <-> device transfers of a context's large arrays: cell
-// fields, whose order differs on the two sides (CellOrder), and packet
-// records.
+// cmi_stage.hpp -- host <-> device transfers of a context's cell fields, whose
+// order differs on the two sides (CellOrder).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -52,9 +51,6 @@ class Stage {
                           const CellField *fields, int nfields);
   hipError_t download_cells(int device, hipStream_t st, const CellOrder &o, size_t n,
                             const CellField *fields, int nfields);
-  // Plain copies.
-  hipError_t upload(int device, hipStream_t st, const void *host, void *dev, size_t bytes);
-  hipError_t download(int device, hipStream_t st, const void *dev, void *host, size_t bytes);
 
  private:
   static constexpr int kThreads = 4;            // host threads of a large transfer
