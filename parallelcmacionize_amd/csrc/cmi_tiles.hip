@@ -1101,16 +1101,69 @@ __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
         const bool out = (q & W.guard) != 0u;
         const uint64_t exited_m = ended_m & lane_mask(out);
         const uint64_t abs_m = ended_m & ~exited_m;
+        if (ended) {
+          // the counters' growth, and the cell the packet was absorbed in
+          const uint32_t vis = (walk_sum(W, q, T0, T1, T2) - q_sum0) + (out ? 0u : 1u);
+          my_cross += vis;
+          if (kList) po.crossings[my_pid] += vis;
+        }
         if (abs_m) {
-          w_abs += (uint32_t)__popcll(abs_m);
+          bool again = false;
           if (lane_in(abs_m)) {
             // absorbed: the partial last step, up to the target optical depth
-            // (reemitting kernels deposited it at the absorption and left
-            // tau = 0)
             const float sa = kap_c > 0.f ? tau * __builtin_amdgcn_rcpf(kap_c) : 0.f;
             AccAtomic<Acc>::add(acc_at(cur), sa, fscale);
             t = t + sa;
+            if (kReemit) {
+              // reemitted with probability reemit_p: the lane walks on, in
+              // place of a new record.  Here, for all lanes that were absorbed
+              // since the last refill at once: about 200 instructions, which
+              // inside the walk ran for one or two lanes at a time and kept
+              // its steps from being nested (128^3 cells, 5e6 packets: 4.17 ->
+              // 3.28 ms a transport).
+              const float q0 = fmaf(t, d0, p0), q1 = fmaf(t, d1, p1), q2 = fmaf(t, d2, p2);
+              const u32x4 r = philox4x32_10(
+                  u32x4{__float_as_uint(q0), __float_as_uint(q1), __float_as_uint(q2),
+                        (uint32_t)tile ^ (n_reemit << 24)},
+                  G.reemit_key[0], G.reemit_key[1]);
+              const float k24 = 1.f / 16777216.f;
+              if (((float)(r.x >> 8) + 0.5f) * k24 < G.reemit_p) {
+                // get_random_direction, testDensitySubGrid_omp.cpp:529-545,
+                // and tau = -ln u: FP32 draws on 24-bit uniforms in (0, 1)
+                const int l0 = walk_index(walk_count(q, W.fs[0], T0), d0, T0);
+                const int l1 = walk_index(walk_count(q, W.fs[1], T1), d1, T1);
+                const int l2 = walk_index(walk_count(q, W.fs[2], T2), d2, T2);
+                const float cost = 2.f * (((float)(r.y >> 8) + 0.5f) * k24) - 1.f;
+                const float phi = 6.28318530717958647692f * (((float)(r.z >> 8) + 0.5f) * k24);
+                const float sint = sqrtf(fmaxf(1.f - cost * cost, 0.f));
+                float sp, cp;
+                sincosf(phi, &sp, &cp);
+                d0 = sint * cp * (float)P.unit_scale[0];
+                d1 = sint * sp * (float)P.unit_scale[1];
+                d2 = cost * (float)P.unit_scale[2];
+                tau = -__logf(((float)(r.w >> 8) + 0.5f) * k24);
+                p0 = q0;
+                p1 = q1;
+                p2 = q2;
+                t = 0.f;
+                ++n_reemit;
+                ++my_re;
+                dda_axis(l0, p0, d0, tm0, td0);
+                dda_axis(l1, p1, d1, tm1, td1);
+                dda_axis(l2, p2, d2, tm2, td2);
+                inc0 = walk_inc(W.fs[0], st0, d0);
+                inc1 = walk_inc(W.fs[1], st1, d1);
+                inc2 = walk_inc(W.fs[2], 4, d2);
+                q = walk_state(W, l0, l1, l2, d0, d1, d2, T0, T1, T2);
+                q_sum0 = walk_sum(W, q, T0, T1, T2);
+                cur = q & offmask;
+                again = true;
+              }
+            }
           }
+          const uint64_t again_m = kReemit ? lane_mask(again) : 0ull;
+          w_abs += (uint32_t)__popcll(abs_m & ~again_m);
+          live_m |= again_m;
         }
         // the exit axis is the one whose counter reached its guard bit; the
         // sign of the flight along it is that of its increment's byte stride
@@ -1123,17 +1176,9 @@ __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
         const uint64_t escaped_m = exited_m & lane_mask(((outside >> face) & 1u) != 0u);
         moving_m = exited_m & ~escaped_m;
         w_esc += (uint32_t)__popcll(escaped_m);
-        if (ended) {
-          if (!kReemit) {
-            // the counters' growth, and the cell the packet was absorbed in
-            const uint32_t vis = (walk_sum(W, q, T0, T1, T2) - q_sum0) + (out ? 0u : 1u);
-            my_cross += vis;
-            if (kList) po.crossings[my_pid] += vis;
-          }
-          if (kList) {
-            po.hops[my_pid] += 1;
-            if (!lane_in(moving_m)) po.status[my_pid] = out ? 1 : 0;
-          }
+        if (kList && ended) {
+          po.hops[my_pid] += 1;
+          if (!lane_in(moving_m)) po.status[my_pid] = out ? 1 : 0;
         }
       }
       uint32_t sbase = 0;
@@ -1206,7 +1251,7 @@ __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
           inc1 = walk_inc(W.fs[1], st1, d1);
           inc2 = walk_inc(W.fs[2], 4, d2);
           q = walk_fields(W, l0, l1, l2, d0, d1, d2, T0, T1, T2) | code;
-          if (!kReemit) q_sum0 = walk_sum(W, q, T0, T1, T2);
+          q_sum0 = walk_sum(W, q, T0, T1, T2);
           cur = code;
           kap_c = kap_at(cur);
         }
@@ -1229,105 +1274,28 @@ __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
       //      while records are left for them, else until every lane has ----
       const int nlive0 = __popcll(live_m);
       const int stop_at = next_m ? max(nlive0 - refill_batch, 0) : 0;
-      if (kReemit) {
-        while (__popcll(live_m) > stop_at) {
-          bool on = false;  // lanes that walk on
-          if (lane_in(live_m)) {
-            ++my_cross;
-            bool f;
-            const float tn = fminf(tm0, fminf(tm1, tm2));
-            const float seg = tn - t;
-            const float dtau = seg * kap_c;
-            if (dtau >= tau) {
-              // absorbed in this cell
-              bool again = false;
-              if (kReemit) {
-                const float sa = kap_c > 0.f ? tau * __builtin_amdgcn_rcpf(kap_c) : 0.f;
-                AccAtomic<Acc>::add(acc_at(cur), sa, fscale);
-                t = t + sa;
-                tau = 0.f;
-                const float q0 = fmaf(t, d0, p0), q1 = fmaf(t, d1, p1), q2 = fmaf(t, d2, p2);
-                const u32x4 r = philox4x32_10(
-                    u32x4{__float_as_uint(q0), __float_as_uint(q1), __float_as_uint(q2),
-                          (uint32_t)tile ^ (n_reemit << 24)},
-                    G.reemit_key[0], G.reemit_key[1]);
-                const float k24 = 1.f / 16777216.f;
-                if (((float)(r.x >> 8) + 0.5f) * k24 < G.reemit_p) {
-                  // get_random_direction, testDensitySubGrid_omp.cpp:529-545,
-                  // and tau = -ln u: FP32 draws on 24-bit uniforms in (0, 1)
-                  const int l0 = walk_index(walk_count(q, W.fs[0], T0), d0, T0);
-                  const int l1 = walk_index(walk_count(q, W.fs[1], T1), d1, T1);
-                  const int l2 = walk_index(walk_count(q, W.fs[2], T2), d2, T2);
-                  const float cost = 2.f * (((float)(r.y >> 8) + 0.5f) * k24) - 1.f;
-                  const float phi = 6.28318530717958647692f * (((float)(r.z >> 8) + 0.5f) * k24);
-                  const float sint = sqrtf(fmaxf(1.f - cost * cost, 0.f));
-                  float sp, cp;
-                  sincosf(phi, &sp, &cp);
-                  d0 = sint * cp * (float)P.unit_scale[0];
-                  d1 = sint * sp * (float)P.unit_scale[1];
-                  d2 = cost * (float)P.unit_scale[2];
-                  tau = -__logf(((float)(r.w >> 8) + 0.5f) * k24);
-                  p0 = q0;
-                  p1 = q1;
-                  p2 = q2;
-                  t = 0.f;
-                  ++n_reemit;
-                  ++my_re;
-                  dda_axis(l0, p0, d0, tm0, td0);
-                  dda_axis(l1, p1, d1, tm1, td1);
-                  dda_axis(l2, p2, d2, tm2, td2);
-                  inc0 = walk_inc(W.fs[0], st0, d0);
-                  inc1 = walk_inc(W.fs[1], st1, d1);
-                  inc2 = walk_inc(W.fs[2], 4, d2);
-                  q = walk_state(W, l0, l1, l2, d0, d1, d2, T0, T1, T2);
-                  again = true;
-                }
-              }
-              f = !again;
-            } else {
-              AccAtomic<Acc>::add(acc_at(cur), seg, fscale);
-              tau -= dtau;
-              t = tn;
-              const bool a0 = tm0 == tn;
-              const bool a1 = !a0 && (tm1 == tn);
-              q += a0 ? inc0 : (a1 ? inc1 : inc2);
-              tm0 += a0 ? td0 : 0.f;
-              tm1 += a1 ? td1 : 0.f;
-              tm2 += (!a0 && !a1) ? td2 : 0.f;
-              f = (q & W.guard) != 0u;
-              cur = q & offmask;
-              kap_c = kap_at(cur);  // the next cell, read ahead
-            }
-            on = !f;
-          }
-          const uint64_t on_m = lane_mask(on);
-          ended_m |= live_m & ~on_m;
-          live_m = on_m;
-        }
-      } else {
-        // kPassSteps steps per pass, nested: a lane that finishes in a pass sits
-        // out its remaining steps, and the count of finished lanes and the
-        // loop's mask bookkeeping are paid once per pass.  3 to 10 steps take
-        // the same time within 3 % (256^3, 1e8 packets: 20.8, 20.6, 20.8,
-        // 20.8, 21.5, 21.5 ms at 3, 4, 5, 6, 8, 10).
-        WalkLane w{tm0, tm1, tm2, td0, td1, td2, t, tau, kap_c, q, cur, inc0, inc1, inc2};
-        auto deposit = [&](uint32_t o, float s) { AccAtomic<Acc>::add(acc_at(o), s, fscale); };
-        while (__popcll(live_m) > stop_at) {
-          bool on = false;  // lanes that walk on after the pass
-          if (lane_in(live_m)) walk_steps<kPassSteps>(w, W.guard, offmask, kap_at, deposit, on);
-          const uint64_t on_m = lane_mask(on);
-          ended_m |= live_m & ~on_m;
-          live_m = on_m;
-        }
-        tm0 = w.tm0;
-        tm1 = w.tm1;
-        tm2 = w.tm2;
-        t = w.t;
-        tau = w.tau;
-        kap_c = w.kap;
-        q = w.q;
-        cur = w.cur;
+      // kPassSteps steps per pass, nested: a lane that finishes in a pass sits
+      // out its remaining steps, and the count of finished lanes and the
+      // loop's mask bookkeeping are paid once per pass.  3 to 10 steps take
+      // the same time within 3 % (256^3, 1e8 packets: 20.8, 20.6, 20.8,
+      // 20.8, 21.5, 21.5 ms at 3, 4, 5, 6, 8, 10).
+      WalkLane w{tm0, tm1, tm2, td0, td1, td2, t, tau, kap_c, q, cur, inc0, inc1, inc2};
+      auto deposit = [&](uint32_t o, float s) { AccAtomic<Acc>::add(acc_at(o), s, fscale); };
+      while (__popcll(live_m) > stop_at) {
+        bool on = false;  // lanes that walk on after the pass
+        if (lane_in(live_m)) walk_steps<kPassSteps>(w, W.guard, offmask, kap_at, deposit, on);
+        const uint64_t on_m = lane_mask(on);
+        ended_m |= live_m & ~on_m;
+        live_m = on_m;
       }
+      tm0 = w.tm0;
+      tm1 = w.tm1;
+      tm2 = w.tm2;
+      t = w.t;
+      tau = w.tau;
+      kap_c = w.kap;
+      q = w.q;
+      cur = w.cur;
     }
     __syncthreads();
     // flush the visit: J deposits, face counts
@@ -1890,14 +1858,15 @@ static void launch_process(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
                      LIST ? e->pid[0] : nullptr, LIST ? e->pid[1] : nullptr, po,       \
                      c->d_cnt, prob_cross, R.refill, e->rel)
   // 16^3 tiles at 512 threads (the tuned shape): the kernel specialised to
-  // them, with its LDS block static.  Emission-driven transports without
-  // reemission only: the specialisation's constants cost the packet-list and
-  // reemitting kernels registers (89 and 99 VGPRs against 75 and 86), and
-  // with them a wave per SIMD.
+  // them, with its LDS block static and six waves per SIMD.  Emission-driven
+  // transports; a list's time is in its host copies.  Reemitting ones fit the 80
+  // VGPRs with 40 bytes spilled at the draws (89 VGPRs and five waves without
+  // the bound): 128^3 cells, 5e6 packets 4.52 -> 4.17 ms a transport.
   const bool t16 = R.threads == 512 && G.T[0] == 16 && G.T[1] == 16 && G.T[2] == 16;
   if (G.reemit_p > 0.f) {
     // reemission: emission-driven transports only
     if (R.threads == 256) CMI_PROC(FixAcc, 256, false, true, 0);
+    else if (t16) CMI_PROC(FixAcc, 512, false, true, 16);
     else CMI_PROC(FixAcc, 512, false, true, 0);
     return;
   }

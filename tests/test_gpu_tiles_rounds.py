@@ -61,3 +61,20 @@ def test_list_equals_emission(npackets):
         assert int(cr.sum()) == s["crossings"] and int(hp.sum()) == s["hops"]
         assert abs(s["crossings"] - ref[0]) <= 2 * npackets * 1e-3
         assert abs(ctx.get_fields()[0].sum() / J.sum() - 1) < 1e-5
+
+
+@pytest.mark.parametrize("npackets", [1, 65, 4097, 100000])
+@pytest.mark.parametrize("p", [0.364, 0.95])
+def test_reemission_is_the_same_in_every_kernel(npackets, p):
+    """Reemitted at the refill of a wave: the kernel of 16^3 tiles (512 threads)
+    and the general one (256) draw the same packets' numbers, so counts and J
+    agree bit for bit, whatever the waves' neighbours are."""
+    with _context([48, 32, 64], [3, 2, 4], 2) as ctx:
+        ctx.set_reemission(p)
+        ref, J = _run(ctx, npackets)
+        assert ref[2] + ref[3] == npackets and ref[4] == 0
+        for t in ({"block_threads": 256}, {"block_threads": 256, "chunk_min": 300},
+                  {"chunk_min": 100000}, {"refill_batch": 1}, {"refill_batch": 64}):
+            got, Jg = _run(ctx, npackets, **t)
+            assert got == ref, t
+            assert Jg.tobytes() == J.tobytes(), t
