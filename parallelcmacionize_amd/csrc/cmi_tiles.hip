@@ -22,7 +22,8 @@
 //             segments, and the next round's work descriptors (tile, start,
 //             count) in chunks, smaller ones for rounds with few packets;
 //   place     segment start + visit's base + rank of every survivor -> the
-//             index list the next round gathers packets through.
+//             index list the next round gathers packets through; one launch
+//             with the plan where the rounds are short (tiles_next_kernel).
 //
 // Round 0 has no visits before it: for emitted packets its per-tile counts
 // follow from the source split, so it is planned before the emission, which
@@ -301,7 +302,13 @@ __global__ void tiles_emit_kernel(TileGeo G, const SetSources *__restrict__ S,
 __global__ void tiles_source_hist_kernel(TileGeo G,
                                          const SetSources *__restrict__ S,
                                          uint32_t *__restrict__ hist,
+                                         uint32_t *__restrict__ nonempty,
                                          SrcTile *__restrict__ src_tile) {
+  // the transport starts with an empty histogram
+  for (int t = (int)threadIdx.x; t < G.ntiles; t += blockDim.x) hist[t] = 0u;
+  if (threadIdx.x == 0) *nonempty = 0u;
+  __threadfence();
+  __syncthreads();
   // one thread per source of every problem; a source's problem is the last
   // p with src_begin[p] <= s
   const int ns = S->src_begin[S->nprob];
@@ -407,14 +414,18 @@ __device__ __forceinline__ uint64_t block_exclusive_scan(uint64_t v,
   }
   if (lane == 63) sh[wave] = x;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t acc = 0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
-      const uint64_t t = sh[w];
-      sh[w] = acc;
-      acc += t;
+  if (wave == 0) {
+    // the waves' sums (at most 16), scanned by the first wave
+    const int nw = (int)(blockDim.x >> 6);
+    const uint64_t w = lane < nw ? sh[lane] : 0;
+    uint64_t y = w;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) {
+      const uint64_t z = __shfl_up(y, off, 64);
+      if (lane >= off) y += z;
     }
-    sh[16] = acc;
+    if (lane < nw) sh[lane] = y - w;
+    if (lane == nw - 1) sh[16] = y;
   }
   __syncthreads();
   const uint64_t r = sh[wave] + x - v;
@@ -435,24 +446,42 @@ static const uint32_t kChunkFloor = 256;  // smallest chunk accepted
 // largest: its 32-byte records stay within 32-bit offsets
 static const uint32_t kChunkMost = 1u << 26;
 
-// total[0]: packets of the round being planned (in: those of the round just
-// processed, kept in total[1]); ndesc[0]: its visits (those of the round just
-// processed are kept in ndesc[1] for the placement); nonempty (optional) counts
-// the plans that found packets.  A round's chunk is `chunk`, or smaller when
-// the round holds fewer than min_visits * chunk packets: then the chunk is cut
-// (down to kChunkFloor) so that the round still has about min_visits visits.
+// What a plan reads and writes.  A round's histogram and visit count have two
+// places, used in turn (TilesEngine::turn): a plan reads `hist`, empties `hist_next`,
+// which the planned round's process kernel adds to, and leaves the visit count
+// in `ndesc`.  total: the packets of the round being planned; nonempty (optional)
+// counts the plans that found packets.  A round's chunk is `chunk`, or smaller
+// when the round holds fewer than min_visits * chunk packets: then the chunk is
+// cut (down to kChunkFloor) so that the round still has about min_visits visits.
 // Late rounds hold few packets; at full chunks they occupy a fraction of the
 // GPU's workgroup slots and the round's time is that of its largest visits,
 // which walk several packets per lane one after the other.
-__global__ void __launch_bounds__(kPlanThreads) tiles_plan_kernel(
-    int ntiles, uint32_t *__restrict__ hist, uint32_t *__restrict__ seg,
-    uint32_t *__restrict__ cursor, Desc *__restrict__ desc,
-    uint32_t *__restrict__ ndesc, uint32_t *__restrict__ total,
-    unsigned *__restrict__ ticket, uint32_t chunk, uint32_t min_visits,
-    const uint16_t *__restrict__ tile_prob, int nprob,
-    uint32_t *__restrict__ prob_round,
-    unsigned long long *__restrict__ prob_time,
-    uint32_t *__restrict__ round_ctr, uint32_t *__restrict__ nonempty) {
+struct PlanArgs {
+  int ntiles;
+  const uint32_t *hist;
+  uint32_t *hist_next, *seg, *cursor;
+  Desc *desc;
+  uint32_t *ndesc, *total;
+  unsigned *ticket;
+  uint32_t chunk, min_visits;
+  const uint16_t *tile_prob;
+  int nprob;
+  uint32_t *prob_round;  // null: no completion marks
+  unsigned long long *prob_time;
+  uint32_t *round_ctr, *nonempty;
+};
+
+// The plan, by one workgroup of kPlanThreads.
+__device__ __forceinline__ void plan_round(const PlanArgs &A) {
+  const int ntiles = A.ntiles;
+  const uint32_t *const hist = A.hist;
+  uint32_t *const seg = A.seg, *const cursor = A.cursor;
+  Desc *const desc = A.desc;
+  uint32_t chunk = A.chunk;
+  const uint32_t min_visits = A.min_visits;
+  const uint16_t *const tile_prob = A.tile_prob;
+  const int nprob = A.nprob;
+  uint32_t *const prob_round = A.prob_round;
   __shared__ uint64_t sh[17];
   __shared__ uint32_t s_pc[kMaxProblems];
   __shared__ uint32_t s_round;
@@ -460,11 +489,7 @@ __global__ void __launch_bounds__(kPlanThreads) tiles_plan_kernel(
   __shared__ uint4 s_crowded[kPlanCrowded];  // tile, first descriptor, count, segment start
   __shared__ uint32_t s_cpre[kPlanCrowded];  // exclusive prefix of their chunks
   const bool track = prob_round != nullptr;
-  if (threadIdx.x == 0) {
-    total[1] = total[0];
-    ndesc[1] = ndesc[0];
-    s_ncrowded = 0;
-  }
+  if (threadIdx.x == 0) s_ncrowded = 0;
   if (track)
     for (int q = threadIdx.x; q < nprob; q += kPlanThreads) s_pc[q] = 0;
   __syncthreads();
@@ -511,7 +536,7 @@ __global__ void __launch_bounds__(kPlanThreads) tiles_plan_kernel(
   auto pass3 = [&](int t, uint32_t c) {
     seg[t] = (uint32_t)base_c;
     cursor[t] = 0;
-    hist[t] = 0;
+    A.hist_next[t] = 0;
     const uint32_t nch = (c + chunk - 1) / chunk;
     uint32_t slot = kPlanCrowded;
     if (nch > kPlanSerialChunks) slot = atomicAdd(&s_ncrowded, 1u);
@@ -565,27 +590,30 @@ __global__ void __launch_bounds__(kPlanThreads) tiles_plan_kernel(
     }
   }
   if (threadIdx.x == 0) {
-    *ndesc = (uint32_t)tot_d;
-    total[0] = (uint32_t)tot_c;
-    *ticket = 0;
-    if (nonempty && tot_c) *nonempty += 1u;
+    *A.ndesc = (uint32_t)tot_d;
+    A.total[0] = (uint32_t)tot_c;
+    *A.ticket = 0;
+    if (A.nonempty && tot_c) *A.nonempty += 1u;
   }
   if (track) {
     // completion of each problem: the first plan that finds it empty
     if (threadIdx.x == 0) {
-      s_round = *round_ctr;
-      *round_ctr = s_round + 1;
+      s_round = *A.round_ctr;
+      *A.round_ctr = s_round + 1;
     }
     __syncthreads();
     const unsigned long long now = wall_clock64();
     for (int q = threadIdx.x; q < nprob; q += kPlanThreads) {
       if (s_pc[q] == 0 && prob_round[q] == kNone) {
         prob_round[q] = s_round;
-        prob_time[q] = now;
+        A.prob_time[q] = now;
       }
     }
   }
 }
+
+// A plan without a placement: round 0's, and those beside tiles_place_kernel.
+__global__ void __launch_bounds__(kPlanThreads) tiles_plan_kernel(PlanArgs A) { plan_round(A); }
 
 // Start of a set iteration: per-problem completion marks cleared, the round
 // counter zeroed and the start time taken.
@@ -682,17 +710,19 @@ __global__ void __launch_bounds__(kScatterThreads) tiles_scatter_kernel(
 // tile and a finished position per slot instead, written and rewritten by the
 // process kernel and read here, 256^3, 1e8 packets took 26.4 ms a transport;
 // with the visits' tables 24.7.
-constexpr int kPlaceThreads = 256;
+constexpr int kPlaceThreads = kPlanThreads;
 constexpr uint32_t kPlacePiece = 4096;
 constexpr uint32_t kRankMask = (1u << 29) - 1u;
 
-__global__ void __launch_bounds__(kPlaceThreads) tiles_place_kernel(
-    const uint32_t *__restrict__ nvisits_ptr, uint32_t pieces_per_visit,
-    const VisitOut *__restrict__ visits, const uint32_t *__restrict__ rel,
-    const uint32_t *__restrict__ seg, uint32_t *__restrict__ idx) {
+// The pieces first, first + stride, ... of the visits; seg: the next round's
+// segments.
+__device__ __forceinline__ void place_pieces(uint32_t first, uint32_t stride, uint32_t items,
+                                             uint32_t pieces_per_visit,
+                                             const VisitOut *__restrict__ visits,
+                                             const uint32_t *__restrict__ rel,
+                                             const uint32_t *seg, uint32_t *__restrict__ idx) {
   __shared__ uint32_t s_at[6];
-  const uint32_t items = *nvisits_ptr * pieces_per_visit;
-  for (uint32_t item = blockIdx.x; item < items; item += gridDim.x) {
+  for (uint32_t item = first; item < items; item += stride) {
     const uint32_t v = item / pieces_per_visit;
     const uint32_t i0 = (item - v * pieces_per_visit) * kPlacePiece;
     const uint32_t ns = visits[v].ns, start = visits[v].start;
@@ -704,21 +734,73 @@ __global__ void __launch_bounds__(kPlaceThreads) tiles_place_kernel(
     }
     __syncthreads();
     const uint32_t i1 = min(ns, i0 + kPlacePiece);
-    constexpr int kAhead = 8;
-    for (uint32_t i = i0 + threadIdx.x; i < i1; i += kAhead * kPlaceThreads) {
-      uint32_t r[kAhead];
+    constexpr int kAhead = kPlacePiece / kPlaceThreads;
+    const uint32_t i = i0 + threadIdx.x;
+    uint32_t r[kAhead];
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) {
-        const uint32_t j = i + (uint32_t)k * kPlaceThreads;
-        r[k] = j < i1 ? rel[start + j] : 0u;
-      }
+    for (int k = 0; k < kAhead; ++k) {
+      const uint32_t j = i + (uint32_t)k * kPlaceThreads;
+      r[k] = j < i1 ? rel[start + j] : 0u;
+    }
 #pragma unroll
-      for (int k = 0; k < kAhead; ++k) {
-        const uint32_t j = i + (uint32_t)k * kPlaceThreads;
-        if (j < i1) idx[s_at[r[k] >> 29] + (r[k] & kRankMask)] = start + j;
-      }
+    for (int k = 0; k < kAhead; ++k) {
+      const uint32_t j = i + (uint32_t)k * kPlaceThreads;
+      if (j < i1) idx[s_at[r[k] >> 29] + (r[k] & kRankMask)] = start + j;
     }
   }
+}
+
+__global__ void __launch_bounds__(kPlaceThreads) tiles_place_kernel(
+    const uint32_t *__restrict__ nvisits, uint32_t pieces_per_visit,
+    const VisitOut *__restrict__ visits, const uint32_t *__restrict__ rel,
+    const uint32_t *__restrict__ seg, uint32_t *__restrict__ idx) {
+  place_pieces(blockIdx.x, gridDim.x, *nvisits * pieces_per_visit, pieces_per_visit, visits, rel,
+               seg, idx);
+}
+
+// Plan and placement of a round in one launch: the first workgroup plans, the
+// others place, each from the segments that it scans itself (in LDS, one word
+// a tile; the planned ones are not there yet).  It is a launch and a single
+// workgroup's latency less per round, where the rounds are short: 64^3 cells,
+// 1e6 packets 0.360 -> 0.341 ms a transport, 128^3, 5e6 with reemission 3.26 ->
+// 3.04, 256^3, 1e7 3.38 -> 3.35; one place workgroup per CU (0.350 and 3.09 with
+// two).  Of rounds of many packets the placement's own time is what counts, and
+// the scans add to it: 256^3, 1e8 packets 20.6 -> 20.8 ms.  So up to
+// kNextPackets packets, and up to kNextTiles tiles, a few reads a thread and 32 KB.
+constexpr int kNextTiles = 8192;
+constexpr size_t kNextPackets = 1u << 25;
+__global__ void __launch_bounds__(kPlanThreads) tiles_next_kernel(
+    PlanArgs A, const uint32_t *__restrict__ nvisits, uint32_t pieces_per_visit,
+    const VisitOut *__restrict__ visits, const uint32_t *__restrict__ rel,
+    uint32_t *__restrict__ idx) {
+  if (blockIdx.x == 0) {
+    plan_round(A);
+    return;
+  }
+  extern __shared__ __align__(16) unsigned char dyn[];
+  uint32_t *const s_seg = reinterpret_cast<uint32_t *>(dyn);
+  __shared__ uint64_t sh[17];
+  const uint32_t items = *nvisits * pieces_per_visit;
+  if (blockIdx.x - 1 >= items) return;
+  constexpr int kPer = kNextTiles / kPlanThreads;
+  const int per = (A.ntiles + kPlanThreads - 1) / kPlanThreads;  // at most kPer
+  const int t0 = (int)threadIdx.x * per;
+  uint32_t c[kPer];
+  uint64_t sum = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    c[k] = k < per && t0 + k < A.ntiles ? A.hist[t0 + k] : 0u;
+    sum += c[k];
+  }
+  uint64_t all;
+  uint32_t at = (uint32_t)block_exclusive_scan(sum, sh, &all);
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    if (k < per && t0 + k < A.ntiles) s_seg[t0 + k] = at;
+    at += c[k];
+  }
+  __syncthreads();
+  place_pieces(blockIdx.x - 1, gridDim.x - 1, items, pieces_per_visit, visits, rel, s_seg, idx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1578,7 +1660,10 @@ struct TilesEngine {
   uint32_t *pid[2] = {nullptr, nullptr};
   uint32_t *idx = nullptr;
   uint32_t *rel = nullptr;      // survivors' positions in their next segment
+  // two histograms and two visit counts, used in turn by the rounds of a
+  // transport: the round's own are hist + turn * ntiles and ndesc + turn
   uint32_t *hist = nullptr, *seg = nullptr, *cursor = nullptr;
+  int turn = 0;
   Desc *desc = nullptr;        // work descriptors of the round
   uint32_t *ndesc = nullptr;
   // [3]: packets of the round being planned, packets of the round just
@@ -1743,7 +1828,7 @@ static int ensure_engine(cmi_ctx *c, const std::vector<ProbGeo> &probs,
   if (err == hipSuccess) err = hipMalloc(&e->visits, e->desc_cap * sizeof(VisitOut));
   if (err == hipSuccess) err = hipMalloc(&e->idx, cap * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->rel, cap * sizeof(uint32_t));
-  if (err == hipSuccess) err = hipMalloc(&e->hist, ntiles * sizeof(uint32_t));
+  if (err == hipSuccess) err = hipMalloc(&e->hist, 2 * (size_t)ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->seg, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->cursor, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->desc, e->desc_cap * sizeof(Desc));
@@ -1781,8 +1866,6 @@ static int ensure_engine(cmi_ctx *c, const std::vector<ProbGeo> &probs,
     free_engine(e);
     return fail(c, CMI_ERR_HIP, "tiles engine: set-up copy failed");
   }
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(64), dim3(256), 0, c->stream, e->hist,
-                     (size_t)ntiles);
   const int max_rounds = max_rounds_of(probs) + 2;
   e->ev.resize(2 * (size_t)max_rounds, nullptr);
   for (hipEvent_t &v : e->ev) {
@@ -1804,6 +1887,7 @@ struct RoundCfg {
   size_t lds;
   unsigned scatter_blocks;
   unsigned place_blocks;
+  bool fused;  // plan and placement in one launch
 };
 
 static RoundCfg round_cfg(const cmi_ctx *c, const TileGeo &G, size_t n0) {
@@ -1843,7 +1927,8 @@ static RoundCfg round_cfg(const cmi_ctx *c, const TileGeo &G, size_t n0) {
                                : (uint32_t)((size_t)r.grid * r.threads));
   const size_t per_block = (size_t)kScatterThreads * kScatterItems;
   r.scatter_blocks = (unsigned)std::min<size_t>(8192, (n0 + per_block - 1) / per_block + 1);
-  r.place_blocks = (unsigned)std::min<size_t>(8 * c->num_cus, n0 / 1024 + 1);
+  r.fused = G.ntiles <= kNextTiles && n0 <= kNextPackets;
+  r.place_blocks = (unsigned)std::min<size_t>((r.fused ? 1 : 2) * c->num_cus, n0 / 1024 + 1);
   return r;
 }
 
@@ -1854,7 +1939,8 @@ static void launch_process(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
 #define CMI_PROC(ACC, TH, LIST, RE, TL)                                            \
   hipLaunchKernelGGL((tiles_process_kernel<ACC, TH, LIST, RE, TL>), dim3(R.grid), dim3(TH), \
                      (TL) ? 0 : R.lds, c->stream, G, c->f.kappa, c->f.J, e->desc,      \
-                     e->ndesc, e->ticket, e->P[0], e->idx, e->P[1], e->visits, e->hist, \
+                     e->ndesc + e->turn, e->ticket, e->P[0], e->idx, e->P[1], e->visits, \
+                     e->hist + (size_t)e->turn * G.ntiles,                             \
                      LIST ? e->pid[0] : nullptr, LIST ? e->pid[1] : nullptr, po,       \
                      c->d_cnt, prob_cross, R.refill, e->rel)
   // 16^3 tiles at 512 threads (the tuned shape): the kernel specialised to
@@ -1906,29 +1992,61 @@ static void launch_walkout(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
 #undef CMI_WALKOUT
 }
 
-// nonempty: count the plans that find packets (total[2]) — the rounds after
-// round 0 that had work.
-static void launch_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
-                        bool track, bool nonempty = false) {
+// Arguments of the next plan, which takes the turn.  nonempty: count the plans
+// that find packets (total[2]) -- the rounds after round 0 that had work.
+static PlanArgs next_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool track,
+                          bool nonempty) {
   TilesEngine *e = c->tiles;
-  hipLaunchKernelGGL(tiles_plan_kernel, dim3(1), dim3(kPlanThreads), 0, c->stream,
-                     G.ntiles, e->hist, e->seg, e->cursor, e->desc, e->ndesc,
-                     e->total, e->ticket, R.chunk, R.min_visits, e->d_tile_prob, e->nprob,
-                     track ? e->d_prob_round : nullptr, e->d_prob_time,
-                     e->d_round_ctr, nonempty ? e->total + 2 : nullptr);
+  PlanArgs A{};
+  A.ntiles = G.ntiles;
+  A.hist = e->hist + (size_t)e->turn * G.ntiles;
+  e->turn ^= 1;
+  A.hist_next = e->hist + (size_t)e->turn * G.ntiles;
+  A.seg = e->seg;
+  A.cursor = e->cursor;
+  A.desc = e->desc;
+  A.ndesc = e->ndesc + e->turn;
+  A.total = e->total;
+  A.ticket = e->ticket;
+  A.chunk = R.chunk;
+  A.min_visits = R.min_visits;
+  A.tile_prob = e->d_tile_prob;
+  A.nprob = e->nprob;
+  A.prob_round = track ? e->d_prob_round : nullptr;
+  A.prob_time = e->d_prob_time;
+  A.round_ctr = e->d_round_ctr;
+  A.nonempty = nonempty ? e->total + 2 : nullptr;
+  return A;
 }
 
-// The placement of a planned round's packets: the survivors of the one before.
-static void launch_place(cmi_ctx *c, const RoundCfg &R) {
+// Plan of round 0, from the histogram of the transport's first turn.
+static void launch_first_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool track) {
+  hipLaunchKernelGGL(tiles_plan_kernel, dim3(1), dim3(kPlanThreads), 0, c->stream,
+                     next_plan(c, G, R, track, false));
+}
+
+// Plan of the next round and placement of its packets, the survivors of the
+// one just processed.
+static void launch_next(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool track,
+                        bool nonempty) {
   TilesEngine *e = c->tiles;
+  const uint32_t *nvisits = e->ndesc + e->turn;
+  const PlanArgs A = next_plan(c, G, R, track, nonempty);
+  const uint32_t pieces = (R.chunk + kPlacePiece - 1) / kPlacePiece;
+  if (R.fused) {
+    hipLaunchKernelGGL(tiles_next_kernel, dim3(R.place_blocks + 1), dim3(kPlanThreads),
+                       G.ntiles * sizeof(uint32_t), c->stream, A, nvisits, pieces, e->visits,
+                       e->rel, e->idx);
+    return;
+  }
+  hipLaunchKernelGGL(tiles_plan_kernel, dim3(1), dim3(kPlanThreads), 0, c->stream, A);
   hipLaunchKernelGGL(tiles_place_kernel, dim3(R.place_blocks), dim3(kPlaceThreads), 0,
-                     c->stream, e->ndesc + 1, (R.chunk + kPlacePiece - 1) / kPlacePiece,
-                     e->visits, e->rel, e->seg, e->idx);
+                     c->stream, nvisits, pieces, e->visits, e->rel, e->seg, e->idx);
 }
 
 // The host checks the packets left every kRoundsPerCheck rounds: a check
 // costs a host round trip (about 30 us), a round launched after the last
-// packet has gone about 20 us (its kernels find no work).
+// packet has gone two launches that find no work.
 constexpr int kRoundsPerCheck = 8;
 
 // Rounds of process / plan / place until no packet is left.  On entry round
@@ -1941,8 +2059,6 @@ static int run_rounds(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool with
   // so their rounds are bounded only by the cap
   const int max_rounds = G.reemit_p > 0.f ? kReemitRoundCap : max_rounds_of(e->probs) + 2;
   const int timed = c->kernel_timing ? std::min<int>(max_rounds, (int)(e->ev.size() / 2)) : 0;
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, c->stream, e->total + 2,
-                     (size_t)1);
   int r = 0;
   bool drained = false;
   if (n0 <= R.finish_max) {
@@ -1959,8 +2075,7 @@ static int run_rounds(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool with
       launch_process(c, G, R, with_pid, po, nullptr);
       if (r < timed) CMI_TRY_HIP(c, hipEventRecord(e->ev[2 * r + 1], c->stream));
       CMI_TRY_HIP(c, hipGetLastError());
-      launch_plan(c, G, R, false, true);
-      launch_place(c, R);
+      launch_next(c, G, R, false, true);
       CMI_TRY_HIP(c, hipGetLastError());
       std::swap(e->P[0], e->P[1]);
       if (with_pid) std::swap(e->pid[0], e->pid[1]);
@@ -2049,9 +2164,10 @@ int tiles_transport(cmi_ctx *c, uint64_t npackets, uint64_t seed,
   CMI_TRY_HIP(c, hipEventRecord(c->ev0, c->stream));
   // round 0: per-tile counts from the source split, planned, then the
   // emission fills the records and the index list
+  e->turn = 0;
   hipLaunchKernelGGL(tiles_source_hist_kernel, dim3(1), dim3(256), 0, c->stream, G,
-                     e->d_src, e->hist, e->src_tile);
-  launch_plan(c, G, R, false);
+                     e->d_src, e->hist, e->total + 2, e->src_tile);
+  launch_first_plan(c, G, R, false);
   const unsigned eb = (unsigned)((npackets + 255) / 256);
   hipLaunchKernelGGL(tiles_emit_kernel, dim3(eb), dim3(256), 0, c->stream, G, e->d_src,
                      npackets, e->P[0], e->seg, e->src_tile, e->idx);
@@ -2121,6 +2237,11 @@ int tiles_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub
     cleanup();
     return fail(c, CMI_ERR_HIP, "tiles list transport: event record failed");
   }
+  e->turn = 0;
+  hipLaunchKernelGGL(zero_u32_kernel, dim3(64), dim3(256), 0, c->stream, e->hist,
+                     (size_t)G.ntiles);
+  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, c->stream, e->total + 2,
+                     (size_t)1);
   hipLaunchKernelGGL(tiles_load_list_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256),
                      0, c->stream, G, c->g, dp, ds, n, e->P[0], e->dest, e->pid[0],
                      e->hist);
@@ -2130,7 +2251,7 @@ int tiles_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub
     return fail(c, CMI_ERR_ARG, "tiles engine: the tile's opacity and accumulator exceed the LDS");
   }
   // round 0: planned from the loaded histogram, index list by destination
-  launch_plan(c, G, R, false);
+  launch_first_plan(c, G, R, false);
   hipLaunchKernelGGL(tiles_scatter_kernel, dim3(R.scatter_blocks), dim3(kScatterThreads),
                      0, c->stream, e->total, e->dest, e->seg, e->cursor, e->idx);
   PacketOut po{dst, dc, dh, fa, fb, dtile};

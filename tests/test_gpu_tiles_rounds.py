@@ -78,3 +78,22 @@ def test_reemission_is_the_same_in_every_kernel(npackets, p):
             got, Jg = _run(ctx, npackets, **t)
             assert got == ref, t
             assert Jg.tobytes() == J.tobytes(), t
+
+
+@pytest.mark.parametrize("ncell", [[64, 64, 128], [64, 64, 132], [4, 4, 4], [4, 8, 12],
+                                   [128, 32, 36]])
+def test_plans_of_many_tiles(ncell):
+    """4^3 tiles: 8192 and 8448 of them (plan and placement in one launch and in
+    two), 1, 6 and 2304 (a thread's tiles not all in range), against the same
+    packets walked out by one launch."""
+    rng = np.random.default_rng(sum(ncell))
+    n = int(np.prod(ncell))
+    with cmi.Context(W.box_10pc(), ncell, [1, 1, 1], cmi.PREC_FP32) as ctx:
+        ctx.set_fields(1e8 * np.exp(rng.normal(0, 1, n)), 10 ** rng.uniform(-6, -2.5, n))
+        ctx.set_sources(rng.uniform(-4 * W.PC, 4 * W.PC, (3, 3)), np.full(3, 1e48))
+        ref, J = _run(ctx, 30000, tile=[4, 4, 4], finish_packets=30000)
+        assert ref[2] + ref[3] == 30000 and ref[4] == 0
+        for t in ({}, {"finish_packets": -1}, {"finish_packets": -1, "chunk_min": 300}):
+            got, Jg = _run(ctx, 30000, tile=[4, 4, 4], **t)
+            assert got == ref, t
+            assert Jg.tobytes() == J.tobytes(), t
