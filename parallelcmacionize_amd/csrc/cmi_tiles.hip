@@ -14,10 +14,10 @@
 //             LDS copy of the tile's J (fixed-point integers, exact in any
 //             order) that is flushed to HBM once per visit;
 //             survivors are written to the workgroup's own output region
-//             (LDS-counter compaction) with their destination tile; the
-//             per-face exit counts go to the next round's tile histogram
-//             (whose old values are the visit's bases) and every survivor
-//             keeps its exit face and its rank among the visit's exits there;
+//             (LDS-counter compaction, grouped by exit face), each with its
+//             exit face and its rank among the visit's exits there; the
+//             per-face exit counts go to the next round's tile histogram,
+//             whose old values are the visit's bases;
 //   plan      one workgroup: exclusive scan of the histogram into tile
 //             segments, and the next round's work descriptors (tile, start,
 //             count) in chunks, smaller ones for rounds with few packets;
@@ -1687,7 +1687,7 @@ struct TilesEngine {
   VisitOut *visits = nullptr;
   uint32_t *pid[2] = {nullptr, nullptr};
   uint32_t *idx = nullptr;
-  uint32_t *rel = nullptr;      // survivors' positions in their next segment
+  uint32_t *rel = nullptr;      // survivors' exit faces and ranks
   // two histograms and two visit counts, used in turn by the rounds of a
   // transport: the round's own are hist + turn * ntiles and ndesc + turn
   uint32_t *hist = nullptr, *seg = nullptr, *cursor = nullptr;
