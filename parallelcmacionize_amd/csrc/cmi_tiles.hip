@@ -42,6 +42,7 @@
 #include <string.h>
 
 #include "cmi_ctx.hpp"
+#include "cmi_place.hpp"
 
 namespace cmi {
 
@@ -175,6 +176,11 @@ struct Desc {
   uint32_t start;
   uint32_t count;
   uint32_t pad;
+};
+
+// A planned round: its visits (descriptors) and the chunk that they were cut to.
+struct Round {
+  uint32_t visits, chunk;
 };
 
 // What a visit leaves for the placement of its survivors (slots start ..
@@ -446,10 +452,9 @@ static const uint32_t kChunkFloor = 256;  // smallest chunk accepted
 // largest: its 32-byte records stay within 32-bit offsets
 static const uint32_t kChunkMost = 1u << 26;
 
-// What a plan reads and writes.  A round's histogram and visit count have two
+// What a plan reads and writes.  A round's histogram and its Round have two
 // places, used in turn (TilesEngine::turn): a plan reads `hist`, empties `hist_next`,
-// which the planned round's process kernel adds to, and leaves the visit count
-// in `ndesc`.  total: the packets of the round being planned; nonempty (optional)
+// which the planned round's process kernel adds to, and fills `round`.  total: the packets of the round being planned; nonempty (optional)
 // counts the plans that found packets.  A round's chunk is `chunk`, or smaller
 // when the round holds fewer than min_visits * chunk packets: then the chunk is
 // cut (down to kChunkFloor) so that the round still has about min_visits visits.
@@ -461,7 +466,8 @@ struct PlanArgs {
   const uint32_t *hist;
   uint32_t *hist_next, *seg, *cursor;
   Desc *desc;
-  uint32_t *ndesc, *total;
+  Round *round;
+  uint32_t *total;
   unsigned *ticket;
   uint32_t chunk, min_visits;
   const uint16_t *tile_prob;
@@ -590,7 +596,7 @@ __device__ __forceinline__ void plan_round(const PlanArgs &A) {
     }
   }
   if (threadIdx.x == 0) {
-    *A.ndesc = (uint32_t)tot_d;
+    *A.round = Round{(uint32_t)tot_d, chunk};
     A.total[0] = (uint32_t)tot_c;
     *A.ticket = 0;
     if (A.nonempty && tot_c) *A.nonempty += 1u;
@@ -705,27 +711,24 @@ __global__ void __launch_bounds__(kScatterThreads) tiles_scatter_kernel(
 // slot its exit face and its rank among its visit's exits through that face,
 // and the visit's neighbour and base per face (reserved by the histogram
 // atomic).  With the segments of the next round planned, the index list is one
-// streaming pass without atomics, 4 B read and 4 B written per survivor, a
-// piece of kPlacePiece slots of a visit to a workgroup.  With a destination
+// streaming pass without atomics, 4 B read and 4 B written per survivor, the
+// visits shared out by place_share.  With a destination
 // tile and a finished position per slot instead, written and rewritten by the
 // process kernel and read here, 256^3, 1e8 packets took 26.4 ms a transport;
 // with the visits' tables 24.7.
 constexpr int kPlaceThreads = kPlanThreads;
-constexpr uint32_t kPlacePiece = 4096;
 constexpr uint32_t kRankMask = (1u << 29) - 1u;
 
-// The pieces first, first + stride, ... of the visits; seg: the next round's
-// segments.
-__device__ __forceinline__ void place_pieces(uint32_t first, uint32_t stride, uint32_t items,
-                                             uint32_t pieces_per_visit,
-                                             const VisitOut *__restrict__ visits,
-                                             const uint32_t *__restrict__ rel,
-                                             const uint32_t *seg, uint32_t *__restrict__ idx) {
+// A workgroup's share of a round's survivors; seg: the next round's segments.
+__device__ __forceinline__ void place_survivors(const PlaceShare &S, uint32_t nvisits,
+                                                const VisitOut *__restrict__ visits,
+                                                const uint32_t *__restrict__ rel,
+                                                const uint32_t *seg,
+                                                uint32_t *__restrict__ idx) {
   __shared__ uint32_t s_at[6];
-  for (uint32_t item = first; item < items; item += stride) {
-    const uint32_t v = item / pieces_per_visit;
-    const uint32_t i0 = (item - v * pieces_per_visit) * kPlacePiece;
+  for (uint32_t v = S.visit; v < nvisits; v += S.visit_step) {
     const uint32_t ns = visits[v].ns, start = visits[v].start;
+    uint32_t i0 = S.part * kPlacePiece;
     if (i0 >= ns) continue;
     __syncthreads();
     if (threadIdx.x < 6) {
@@ -733,29 +736,31 @@ __device__ __forceinline__ void place_pieces(uint32_t first, uint32_t stride, ui
       s_at[threadIdx.x] = t == kNone ? 0u : seg[t] + visits[v].base[threadIdx.x];
     }
     __syncthreads();
-    const uint32_t i1 = min(ns, i0 + kPlacePiece);
-    constexpr int kAhead = kPlacePiece / kPlaceThreads;
-    const uint32_t i = i0 + threadIdx.x;
-    uint32_t r[kAhead];
+    for (; i0 < ns; i0 += S.parts * kPlacePiece) {
+      const uint32_t i1 = min(ns, i0 + kPlacePiece);
+      constexpr int kAhead = kPlacePiece / kPlaceThreads;
+      const uint32_t i = i0 + threadIdx.x;
+      uint32_t r[kAhead];
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      const uint32_t j = i + (uint32_t)k * kPlaceThreads;
-      r[k] = j < i1 ? rel[start + j] : 0u;
-    }
+      for (int k = 0; k < kAhead; ++k) {
+        const uint32_t j = i + (uint32_t)k * kPlaceThreads;
+        r[k] = j < i1 ? rel[start + j] : 0u;
+      }
 #pragma unroll
-    for (int k = 0; k < kAhead; ++k) {
-      const uint32_t j = i + (uint32_t)k * kPlaceThreads;
-      if (j < i1) idx[s_at[r[k] >> 29] + (r[k] & kRankMask)] = start + j;
+      for (int k = 0; k < kAhead; ++k) {
+        const uint32_t j = i + (uint32_t)k * kPlaceThreads;
+        if (j < i1) idx[s_at[r[k] >> 29] + (r[k] & kRankMask)] = start + j;
+      }
     }
   }
 }
 
 __global__ void __launch_bounds__(kPlaceThreads) tiles_place_kernel(
-    const uint32_t *__restrict__ nvisits, uint32_t pieces_per_visit,
-    const VisitOut *__restrict__ visits, const uint32_t *__restrict__ rel,
-    const uint32_t *__restrict__ seg, uint32_t *__restrict__ idx) {
-  place_pieces(blockIdx.x, gridDim.x, *nvisits * pieces_per_visit, pieces_per_visit, visits, rel,
-               seg, idx);
+    const Round *__restrict__ round, const VisitOut *__restrict__ visits,
+    const uint32_t *__restrict__ rel, const uint32_t *__restrict__ seg,
+    uint32_t *__restrict__ idx) {
+  place_survivors(place_share(blockIdx.x, gridDim.x, round->chunk), round->visits, visits, rel,
+                  seg, idx);
 }
 
 // Plan and placement of a round in one launch: the first workgroup plans, the
@@ -770,9 +775,8 @@ __global__ void __launch_bounds__(kPlaceThreads) tiles_place_kernel(
 constexpr int kNextTiles = 8192;
 constexpr size_t kNextPackets = 1u << 25;
 __global__ void __launch_bounds__(kPlanThreads) tiles_next_kernel(
-    PlanArgs A, const uint32_t *__restrict__ nvisits, uint32_t pieces_per_visit,
-    const VisitOut *__restrict__ visits, const uint32_t *__restrict__ rel,
-    uint32_t *__restrict__ idx) {
+    PlanArgs A, const Round *__restrict__ round, const VisitOut *__restrict__ visits,
+    const uint32_t *__restrict__ rel, uint32_t *__restrict__ idx) {
   if (blockIdx.x == 0) {
     plan_round(A);
     return;
@@ -780,8 +784,9 @@ __global__ void __launch_bounds__(kPlanThreads) tiles_next_kernel(
   extern __shared__ __align__(16) unsigned char dyn[];
   uint32_t *const s_seg = reinterpret_cast<uint32_t *>(dyn);
   __shared__ uint64_t sh[17];
-  const uint32_t items = *nvisits * pieces_per_visit;
-  if (blockIdx.x - 1 >= items) return;
+  const uint32_t nvisits = round->visits;
+  const PlaceShare share = place_share(blockIdx.x - 1, gridDim.x - 1, round->chunk);
+  if (share.visit >= nvisits) return;
   constexpr int kPer = kNextTiles / kPlanThreads;
   const int per = (A.ntiles + kPlanThreads - 1) / kPlanThreads;  // at most kPer
   const int t0 = (int)threadIdx.x * per;
@@ -800,7 +805,7 @@ __global__ void __launch_bounds__(kPlanThreads) tiles_next_kernel(
     at += c[k];
   }
   __syncthreads();
-  place_pieces(blockIdx.x - 1, gridDim.x - 1, items, pieces_per_visit, visits, rel, s_seg, idx);
+  place_survivors(share, nvisits, visits, rel, s_seg, idx);
 }
 
 // ---------------------------------------------------------------------------
@@ -1030,7 +1035,7 @@ __device__ __forceinline__ void walk_steps(WalkLane &w, uint32_t guard, uint32_t
 template <class Acc, int kThreads, bool kList, bool kReemit = false, int kTile = 0>
 __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
     TileGeo G, const float *__restrict__ kappa, double *__restrict__ J,
-    const Desc *__restrict__ desc, const uint32_t *__restrict__ ndesc_ptr,
+    const Desc *__restrict__ desc, const Round *__restrict__ round,
     unsigned *__restrict__ ticket, const Rec32 *__restrict__ Pin,
     const uint32_t *__restrict__ idx, Rec32 *__restrict__ Pout,
     VisitOut *__restrict__ visit_out, uint32_t *__restrict__ hist_next,
@@ -1081,7 +1086,7 @@ __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
 
   const int lane = threadIdx.x & 63;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  const uint32_t ndesc = *ndesc_ptr;
+  const uint32_t ndesc = round->visits;
   if (blockIdx.x >= ndesc) return;  // no visit for this workgroup
   const int T0 = kTile ? kTile : G.T[0], T1 = kTile ? kTile : G.T[1],
             T2 = kTile ? kTile : G.T[2];
@@ -1688,12 +1693,12 @@ struct TilesEngine {
   uint32_t *pid[2] = {nullptr, nullptr};
   uint32_t *idx = nullptr;
   uint32_t *rel = nullptr;      // survivors' exit faces and ranks
-  // two histograms and two visit counts, used in turn by the rounds of a
-  // transport: the round's own are hist + turn * ntiles and ndesc + turn
+  // two histograms and two Rounds, used in turn by the rounds of a transport:
+  // the round's own are hist + turn * ntiles and round + turn
   uint32_t *hist = nullptr, *seg = nullptr, *cursor = nullptr;
   int turn = 0;
   Desc *desc = nullptr;        // work descriptors of the round
-  uint32_t *ndesc = nullptr;
+  Round *round = nullptr;
   // [3]: packets of the round being planned, packets of the round just
   // processed, number of plans that found packets
   uint32_t *total = nullptr;
@@ -1734,7 +1739,7 @@ static void free_engine(TilesEngine *e) {
   hipFree(e->seg);
   hipFree(e->cursor);
   hipFree(e->desc);
-  hipFree(e->ndesc);
+  hipFree(e->round);
   hipFree(e->total);
   hipFree(e->ticket);
   hipFree(e->src_tile);
@@ -1860,7 +1865,7 @@ static int ensure_engine(cmi_ctx *c, const std::vector<ProbGeo> &probs,
   if (err == hipSuccess) err = hipMalloc(&e->seg, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->cursor, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->desc, e->desc_cap * sizeof(Desc));
-  if (err == hipSuccess) err = hipMalloc(&e->ndesc, 2 * sizeof(uint32_t));
+  if (err == hipSuccess) err = hipMalloc(&e->round, 2 * sizeof(Round));
   if (err == hipSuccess) err = hipMalloc(&e->total, 3 * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->ticket, sizeof(unsigned));
   if (err == hipSuccess) err = hipHostMalloc(&e->h_total, 3 * sizeof(uint32_t));
@@ -1967,7 +1972,7 @@ static void launch_process(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
 #define CMI_PROC(ACC, TH, LIST, RE, TL)                                            \
   hipLaunchKernelGGL((tiles_process_kernel<ACC, TH, LIST, RE, TL>), dim3(R.grid), dim3(TH), \
                      (TL) ? 0 : R.lds, c->stream, G, c->f.kappa, c->f.J, e->desc,      \
-                     e->ndesc + e->turn, e->ticket, e->P[0], e->idx, e->P[1], e->visits, \
+                     e->round + e->turn, e->ticket, e->P[0], e->idx, e->P[1], e->visits, \
                      e->hist + (size_t)e->turn * G.ntiles,                             \
                      LIST ? e->pid[0] : nullptr, LIST ? e->pid[1] : nullptr, po,       \
                      c->d_cnt, prob_cross, R.refill, e->rel)
@@ -2033,7 +2038,7 @@ static PlanArgs next_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool 
   A.seg = e->seg;
   A.cursor = e->cursor;
   A.desc = e->desc;
-  A.ndesc = e->ndesc + e->turn;
+  A.round = e->round + e->turn;
   A.total = e->total;
   A.ticket = e->ticket;
   A.chunk = R.chunk;
@@ -2058,18 +2063,17 @@ static void launch_first_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, b
 static void launch_next(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool track,
                         bool nonempty) {
   TilesEngine *e = c->tiles;
-  const uint32_t *nvisits = e->ndesc + e->turn;
+  const Round *round = e->round + e->turn;
   const PlanArgs A = next_plan(c, G, R, track, nonempty);
-  const uint32_t pieces = (R.chunk + kPlacePiece - 1) / kPlacePiece;
   if (R.fused) {
     hipLaunchKernelGGL(tiles_next_kernel, dim3(R.place_blocks + 1), dim3(kPlanThreads),
-                       G.ntiles * sizeof(uint32_t), c->stream, A, nvisits, pieces, e->visits,
-                       e->rel, e->idx);
+                       G.ntiles * sizeof(uint32_t), c->stream, A, round, e->visits, e->rel,
+                       e->idx);
     return;
   }
   hipLaunchKernelGGL(tiles_plan_kernel, dim3(1), dim3(kPlanThreads), 0, c->stream, A);
   hipLaunchKernelGGL(tiles_place_kernel, dim3(R.place_blocks), dim3(kPlaceThreads), 0,
-                     c->stream, nvisits, pieces, e->visits, e->rel, e->seg, e->idx);
+                     c->stream, round, e->visits, e->rel, e->seg, e->idx);
 }
 
 // The host checks the packets left every kRoundsPerCheck rounds: a check
