@@ -37,4 +37,16 @@ constexpr PlaceShare place_share(uint32_t block, uint32_t blocks, uint32_t chunk
   return PlaceShare{block < step * parts ? block / parts : 0xffffffffu, step, block % parts, parts};
 }
 
+// Workgroups of a placement: one per 1024 packets of the transport, and one
+// per visit that a round of few packets can have (a visit costs its workgroup
+// a chain of loads whatever it holds), up to `most`.  One workgroup for all of
+// 512 visits make an iteration of 64 problems of 8 tiles, 10 packets each,
+// take 0.53 ms instead of 0.28, of 1 packet each 0.38 instead of 0.28.
+constexpr uint32_t place_blocks(uint64_t packets, uint64_t tiles, uint32_t most) {
+  const uint64_t visits = packets < tiles ? packets : tiles;
+  uint64_t blocks = packets / 1024 + 1;
+  if (blocks < visits) blocks = visits;
+  return blocks < most ? (uint32_t)blocks : most;
+}
+
 }  // namespace cmi

@@ -1961,7 +1961,7 @@ static RoundCfg round_cfg(const cmi_ctx *c, const TileGeo &G, size_t n0) {
   const size_t per_block = (size_t)kScatterThreads * kScatterItems;
   r.scatter_blocks = (unsigned)std::min<size_t>(8192, (n0 + per_block - 1) / per_block + 1);
   r.fused = G.ntiles <= kNextTiles && n0 <= kNextPackets;
-  r.place_blocks = (unsigned)std::min<size_t>((r.fused ? 1 : 2) * c->num_cus, n0 / 1024 + 1);
+  r.place_blocks = place_blocks(n0, G.ntiles, (r.fused ? 1 : 2) * c->num_cus);
   return r;
 }
 

@@ -12,10 +12,11 @@ from parallelcmacionize_amd import workloads as W
 HERE = os.path.dirname(os.path.abspath(__file__))
 
 
-def test_every_piece_is_placed_once(tmp_path):
-    exe = str(tmp_path / "place_shares")
+@pytest.mark.parametrize("program", ["place_shares", "place_blocks"])
+def test_shares_and_workgroups(tmp_path, program):
+    exe = str(tmp_path / program)
     subprocess.run(["g++", "-std=c++17", "-O2", "-Wall", "-Werror", "-o", exe,
-                    os.path.join(HERE, "cpp", "place_shares.cpp")], check=True)
+                    os.path.join(HERE, "cpp", program + ".cpp")], check=True)
     r = subprocess.run([exe], capture_output=True, text=True)
     assert r.returncode == 0, r.stdout
 
