@@ -1124,6 +1124,9 @@ __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
       float4 *dst = reinterpret_cast<float4 *>(kapL);
       for (int i = threadIdx.x; i < (tile_cells >> 2); i += kThreads)
         dst[i] = src[i];
+      // tiles of one or two cells are less than a float4
+      if (tile_cells < 4 && (int)threadIdx.x < tile_cells)
+        kapL[threadIdx.x] = kappa[(size_t)tile * tile_cells + threadIdx.x];
       for (int i = threadIdx.x; i < tile_cells; i += kThreads) accL[i] = (Acc)0;
       if (threadIdx.x == 0) {
         s_next = kThreads;  // the first kThreads packets are claimed below
