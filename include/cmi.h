@@ -419,7 +419,8 @@ int cmi_net_get_start_rule(const cmi_net *net, float *logit_cut,
  * opacity refreshed.  cmi_prolong_neutral_fraction: fine x_n = the coarse
  * x_n's logit (clamped to [1e-7, 1 - 1/150]) interpolated trilinearly at
  * each fine cell centre, J = 0, FP32 opacity refreshed.  Each waits for the
- * source context's stream and launches on the destination's. */
+ * source context's stream and launches on the destination's; the source's
+ * stream waits for that launch before what it gets next. */
 int cmi_restrict_density(cmi_ctx *fine, cmi_ctx *coarse);
 int cmi_prolong_neutral_fraction(cmi_ctx *coarse, cmi_ctx *fine);
 /* The same features of a context (by the input mode), as [D][H][W][2] FP32

@@ -391,8 +391,9 @@ int cmi_set_engine(cmi_ctx *c, int engine, const cmi_tuning *t) {
 int cmi_set_fields(cmi_ctx *c, const double *nH, const double *xn) {
   if (!c) return CMI_ERR_ARG;
   (void)hipSetDevice(c->device);
-  // on the context's stream, behind what is queued there (a restriction or
-  // prolongation, a warm start)
+  // on the context's stream, behind what is queued there: a restriction or
+  // prolongation into this context, or out of it (which makes this stream wait
+  // until the other context's has read the fields)
   CMI_TRY_HIP(c, put_fields(c, CellField{const_cast<double *>(nH), c->f.n, 1.},
                             CellField{const_cast<double *>(xn), c->f.xn, 1.}));
   if (c->precision == CMI_PREC_FP32) {

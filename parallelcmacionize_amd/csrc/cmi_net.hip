@@ -1705,6 +1705,18 @@ static int coarse_factor(const cmi_ctx *fine, const cmi_ctx *coarse) {
   return f;
 }
 
+// What is queued on `reader`'s stream reads `source`'s fields: work that
+// `source` gets from here on waits for it.
+static hipError_t hold_fields(cmi_ctx *source, const cmi_ctx *reader) {
+  hipEvent_t read = nullptr;
+  hipError_t e = hipEventCreateWithFlags(&read, hipEventDisableTiming);
+  if (e != hipSuccess) return e;
+  e = hipEventRecord(read, reader->stream);
+  if (e == hipSuccess) e = hipStreamWaitEvent(source->stream, read, 0);
+  const hipError_t d = hipEventDestroy(read);  // released once it has passed
+  return e == hipSuccess ? d : e;
+}
+
 int cmi_restrict_density(cmi_ctx *fine, cmi_ctx *coarse) {
   const int f = coarse_factor(fine, coarse);
   if (!f)
@@ -1723,6 +1735,7 @@ int cmi_restrict_density(cmi_ctx *fine, cmi_ctx *coarse) {
                      coarse->f.xn, coarse->f.J, fp32 ? coarse->f.kappa : (float *)nullptr,
                      coarse->sigma * coarse->g.cell_size[0]);
   CMI_TRY_HIP(coarse, hipGetLastError());
+  CMI_TRY_HIP(coarse, hold_fields(fine, coarse));
   return CMI_OK;
 }
 
@@ -1744,6 +1757,7 @@ int cmi_prolong_neutral_fraction(cmi_ctx *coarse, cmi_ctx *fine) {
                      fp32 ? fine->f.kappa : (float *)nullptr,
                      fine->sigma * fine->g.cell_size[0]);
   CMI_TRY_HIP(fine, hipGetLastError());
+  CMI_TRY_HIP(fine, hold_fields(coarse, fine));
   return CMI_OK;
 }
 
