@@ -1218,6 +1218,7 @@ void input_features(cmi_net *n, const float *feat, int B, const int dim[3]) {
 
 // forward over n->in (B samples of D x H x W) -> zout
 int forward(cmi_net *n, int B, int D, int H, int W, float *zout) {
+  if ((size_t)B * D * H * W == 0) return CMI_OK;  // nothing to compute, no empty grids
   const int nrun = B * D * H * (W / 16);
   const unsigned runs = grid_for((size_t)nrun, 4, 1u << 30);  // one wave per run
   const __bf16 *const in = reinterpret_cast<const __bf16 *>(n->in);
@@ -1277,7 +1278,8 @@ int backward(cmi_net *n, int B, int D, int H, int W) {
                      n->z, n->tgt, nvox, n->w_pos, n->dz, n->g, n->grad_stride, n->nparam,
                      n->off_b[last]);
   __bf16 *dy = n->dact[0], *dx = n->dact[1];
-  for (int l = last; l >= 0; --l) {
+  // without voxels the mean loss is NaN and the gradients stay 0
+  for (int l = nvox ? last : -1; l >= 0; --l) {
     const BlockGeo Gw = block_geo(B, D, H, W, n->dil[l], kGZ);
     const BlockGeo Gx = block_geo(B, D, H, W, n->dil[l], kE);
     const unsigned wg = grad_grid(n, Gw);
@@ -1580,6 +1582,7 @@ int cmi_net_train(cmi_net *n, int steps, int batch, const int crop[3], float lr,
 int cmi_net_loss_and_grad(cmi_net *n, const float *feat, const float *target, int B,
                           const int dim[3], float *loss, float *grad) {
   if (!n || !feat || !target || B <= 0 || !dim) return CMI_ERR_ARG;
+  if (dim[0] < 0 || dim[1] < 0 || dim[2] < 0) return nfail(n, CMI_ERR_ARG, "negative extent");
   if (dim[2] % 32 != 0) return nfail(n, CMI_ERR_ARG, "last extent must be a multiple of 32");
   (void)hipSetDevice(n->device);
   NET_TRY(n, hipStreamSynchronize(n->stream));  // null-stream copies below
@@ -1619,6 +1622,7 @@ int cmi_net_loss_and_grad(cmi_net *n, const float *feat, const float *target, in
 // Logits of x_n for one grid (features [D][H][W][2]).
 int cmi_net_predict(cmi_net *n, const float *feat, const int dim[3], float *logits) {
   if (!n || !feat || !dim || !logits) return CMI_ERR_ARG;
+  if (dim[0] < 0 || dim[1] < 0 || dim[2] < 0) return nfail(n, CMI_ERR_ARG, "negative extent");
   if (dim[2] % 32 != 0) return nfail(n, CMI_ERR_ARG, "last extent must be a multiple of 32");
   (void)hipSetDevice(n->device);
   NET_TRY(n, hipStreamSynchronize(n->stream));  // null-stream copies below
