@@ -371,8 +371,8 @@ int cmi_net_get_dilation(const cmi_net *net, int dilation[4]);
 int cmi_net_set_input_mode(cmi_net *net, int mode);
 int cmi_net_get_input_mode(const cmi_net *net);
 /* Forward convolutions through the kernel that stages blocks of the volume in
- * LDS (on, the default) or through the one that reads every tap from memory;
- * the outputs are identical. */
+ * LDS wherever the volume fills them (on, the default), or always through the
+ * one that reads every tap from memory; the outputs are identical. */
 int cmi_net_set_tiled(cmi_net *net, int on);
 /* weight of the squared logit error where the prediction is more neutral
  * than the target (default 1: plain mean squared error) */

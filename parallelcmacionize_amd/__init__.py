@@ -573,8 +573,8 @@ class WarmStartNet:
 
     def set_tiled(self, on):
         """Forward convolutions through the kernel that stages blocks in LDS
-        (default), or through the per-run kernel; the outputs are
-        identical."""
+        wherever the volume fills them (default), or always through the
+        per-run kernel; the outputs are identical."""
         self._check(self.lib.cmi_net_set_tiled(self.h, int(bool(on))))
 
     def input_mode(self):

@@ -10,8 +10,11 @@
 //                  input gradient (the same convolution over the output
 //                  gradient with the flipped, transposed weights, masked by
 //                  the ReLU of the layer below).
-//   conv3_kernel   the forward convolution without LDS, one wave per run of 16
-//                  voxels (cmi_net_set_tiled(0)): the same outputs bit for bit.
+//   conv3_kernel   the same convolution without LDS, one wave per run of 16
+//                  voxels: for volumes that leave the blocks mostly empty
+//                  (dilations near the volume's edges), and for all forward
+//                  passes after cmi_net_set_tiled(0).  The same outputs bit for
+//                  bit.
 //   wgrad_block_kernel  weight and bias gradient dW[tap][cout][cin] = sum_v
 //                  dy[v][cout] * x[v + tap][cin] on the same MFMA, K = voxels,
 //                  all 27 taps of a workgroup's blocks kept in registers.
@@ -74,7 +77,8 @@ template <int NB, bool kFeat>
 __global__ void __launch_bounds__(256) conv3_kernel(
     const __bf16 *__restrict__ x, const __bf16 *__restrict__ w,
     const float *__restrict__ bias, int nrun, int D, int H, int W, int dil,
-    __bf16 *__restrict__ y, float *__restrict__ yf, int relu) {
+    __bf16 *__restrict__ y, float *__restrict__ yf, const __bf16 *__restrict__ mask,
+    int relu) {
   const int lane = threadIdx.x & 63;
   const int run = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (run >= nrun) return;  // whole wave leaves together
@@ -124,6 +128,7 @@ __global__ void __launch_bounds__(256) conv3_kernel(
     for (int i = 0; i < 4; ++i) {
       const size_t v = vbase + 4 * kg + i;
       float r = acc[nb][i] + (bias ? bias[co] : 0.f);
+      if (mask) r = bf2f(mask[v * kC + co]) > 0.f ? r : 0.f;
       if (relu) r = fmaxf(r, 0.f);
       if (y) y[v * kC + co] = f2bf(r);
       if (yf && co == 0) yf[v] = r;
@@ -140,23 +145,43 @@ __global__ void __launch_bounds__(256) conv3_kernel(
 // past its sub-lattice (zeros in, nothing out).  8^3 rather than rows of 16
 // voxels along the last axis, because the sub-lattices of the 64^3 training
 // crops at dilation 8 are 8^3.
+//
+// Packed blocks (kPack).  Along an axis where a whole sub-lattice has at most 3
+// voxels a block holds several sub-lattices of consecutive residues, one empty
+// position between neighbours: all that a tap past a sub-lattice's end meets is
+// the zero padding, and one position of it serves both.  One sub-lattice a block
+// would fill 1/512 of it at a dilation beyond the volume; packed, an axis is at
+// least half filled.  Four training steps of two 64^3 crops at dilations of 32 and
+// of 64: 35.4 and 253 ms before, 4.4 and 5.8 with packed blocks (and convolutions
+// run by run where those are sparse).
 // ---------------------------------------------------------------------------
 constexpr int kE = 8;        // block edge
 constexpr int kHE = kE + 2;  // with the halo
 
-struct BlockGeo {
-  int D, H, W, dil;
-  int nrz, nry, nrx;  // residues per axis
-  int nbz, nby, nbx;  // blocks per axis of the largest sub-lattice
-  int nblocks;
+// Residues along an axis: `res` of them, `per_block` to a block, each with
+// `period` positions (its voxels and an empty one); inv: 1 / period in 1/256,
+// exact over a block's positions.  Not packed: 1, 0, 0.
+struct Residues {
+  int res, per_block, period, inv;
 };
 
-// One block: its sample, residues, first voxel and sub-lattice extents.
+struct BlockGeo {
+  int D, H, W, dil;
+  int nrz, nry, nrx;  // residues per axis (packed: groups of residues)
+  int nbz, nby, nbx;  // blocks per axis of the largest sub-lattice
+  int nblocks;
+  bool packed;        // some axis has several residues to a block
+  bool sparse;        // convolutions run by run instead (block_geo)
+  Residues pz, py, px;
+};
+
+// One block: its sample, (first) residues, first voxel and the extents of
+// (the first) sub-lattice.
 struct Block {
   int b, rz, ry, rx, z0, y0, x0, Ds, Hs, Ws;
 };
 
-template <int kBZ>
+template <int kBZ, bool kPack>
 __device__ __forceinline__ Block block_of(const BlockGeo &G, int t) {
   Block k;
   k.x0 = (t % G.nbx) * kE;
@@ -171,15 +196,48 @@ __device__ __forceinline__ Block block_of(const BlockGeo &G, int t) {
   t /= G.nry;
   k.rz = t % G.nrz;
   k.b = t / G.nrz;
+  if (kPack) {
+    k.rx *= G.px.per_block;
+    k.ry *= G.py.per_block;
+    k.rz *= G.pz.per_block;
+  }
   k.Ds = (G.D - k.rz + G.dil - 1) / G.dil;
   k.Hs = (G.H - k.ry + G.dil - 1) / G.dil;
   k.Ws = (G.W - k.rx + G.dil - 1) / G.dil;
   return k;
 }
 
-// Voxel number of sub-lattice voxel (sz, sy, sx), or -1 outside the volume.
-__device__ __forceinline__ long long block_voxel(const BlockGeo &G, const Block &k, int sz,
-                                                 int sy, int sx) {
+// Coordinate of a block's position u along a packed axis, or -1 where it holds
+// no voxel of the volume (extent cells).
+__device__ __forceinline__ int packed_coord(const Residues &P, int r0, int x0, int extent,
+                                            int dil, int u) {
+  const int s = (u * P.inv) >> 8;  // which of the block's residues (-1 before the first)
+  const int o = x0 + u - s * P.period;
+  const int c = r0 + s + dil * o;  // past the volume for a residue's empty position
+  return (unsigned)s < (unsigned)min(P.per_block, P.res - r0) && o >= 0 && c < extent ? c : -1;
+}
+// Positions of a block that hold voxels along an axis, as bits.
+__device__ __forceinline__ unsigned packed_positions(const Residues &P, int r0, int x0,
+                                                     int extent, int dil) {
+  unsigned m = 0;
+  for (int u = 0; u < kE; ++u)
+    if (packed_coord(P, r0, x0, extent, dil, u) >= 0) m |= 1u << u;
+  return m;
+}
+
+// Voxel number at position (uz, uy, ux) of a block, counted from its first
+// voxel, or -1 outside the volume.
+template <bool kPack>
+__device__ __forceinline__ long long block_voxel(const BlockGeo &G, const Block &k, int uz,
+                                                 int uy, int ux) {
+  if (kPack) {
+    const int z = packed_coord(G.pz, k.rz, k.z0, G.D, G.dil, uz);
+    const int y = packed_coord(G.py, k.ry, k.y0, G.H, G.dil, uy);
+    const int x = packed_coord(G.px, k.rx, k.x0, G.W, G.dil, ux);
+    if ((z | y | x) < 0) return -1;
+    return ((long long)(k.b * G.D + z) * G.H + y) * G.W + x;
+  }
+  const int sz = k.z0 + uz, sy = k.y0 + uy, sx = k.x0 + ux;
   if ((unsigned)sz >= (unsigned)k.Ds || (unsigned)sy >= (unsigned)k.Hs ||
       (unsigned)sx >= (unsigned)k.Ws)
     return -1;
@@ -187,12 +245,13 @@ __device__ __forceinline__ long long block_voxel(const BlockGeo &G, const Block 
          G.dil * sx;
 }
 // Halo voxel v (of (kBZ + 2) x 10 x 10) and inner voxel o (of kBZ x 8 x 8).
+template <bool kPack>
 __device__ __forceinline__ long long halo_voxel(const BlockGeo &G, const Block &k, int v) {
-  return block_voxel(G, k, k.z0 - 1 + v / (kHE * kHE), k.y0 - 1 + (v / kHE) % kHE,
-                     k.x0 - 1 + v % kHE);
+  return block_voxel<kPack>(G, k, v / (kHE * kHE) - 1, (v / kHE) % kHE - 1, v % kHE - 1);
 }
+template <bool kPack>
 __device__ __forceinline__ long long inner_voxel(const BlockGeo &G, const Block &k, int o) {
-  return block_voxel(G, k, k.z0 + (o >> 6), k.y0 + ((o >> 3) & 7), k.x0 + (o & 7));
+  return block_voxel<kPack>(G, k, o >> 6, (o >> 3) & 7, o & 7);
 }
 
 // ---------------------------------------------------------------------------
@@ -213,7 +272,7 @@ __device__ __forceinline__ long long inner_voxel(const BlockGeo &G, const Block 
 // ---------------------------------------------------------------------------
 constexpr int kConvThreads = 256;
 
-template <int NB, bool kFeat>
+template <int NB, bool kFeat, bool kPack>
 __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
     BlockGeo G, const __bf16 *__restrict__ x, const __bf16 *__restrict__ w,
     const float *__restrict__ bias, __bf16 *__restrict__ y, float *__restrict__ yf,
@@ -222,7 +281,7 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
   constexpr int kInBytes = kHalo * (kFeat ? 4 : 64);
   constexpr int kOutBytes = NB == 2 ? kE * kE * kE * 64 : 0;
   __shared__ __align__(16) unsigned char lds[kInBytes > kOutBytes ? kInBytes : kOutBytes];
-  const Block k = block_of<kE>(G, blockIdx.x);
+  const Block k = block_of<kE, kPack>(G, blockIdx.x);
   if (k.z0 >= k.Ds || k.y0 >= k.Hs || k.x0 >= k.Ws) return;
   // every thread issues all of its loads before its first LDS store, so the
   // block's memory latency is paid once, not once per load
@@ -232,7 +291,7 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int v = (int)threadIdx.x + i * kConvThreads;
-      const long long g = v < kHalo ? halo_voxel(G, k, v) : -1;
+      const long long g = v < kHalo ? halo_voxel<kPack>(G, k, v) : -1;
       vals[i] = g >= 0 ? reinterpret_cast<const uint32_t *>(x)[g] : 0u;
     }
 #pragma unroll
@@ -246,7 +305,7 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
 #pragma unroll
     for (int i = 0; i < kLoads; ++i) {
       const int p = (int)threadIdx.x + i * kConvThreads;  // 16-byte piece
-      const long long g = p < 4 * kHalo ? halo_voxel(G, k, p >> 2) : -1;
+      const long long g = p < 4 * kHalo ? halo_voxel<kPack>(G, k, p >> 2) : -1;
       vals[i] = bf16x8{};
       if (g >= 0) vals[i] = *reinterpret_cast<const bf16x8 *>(x + g * kC + 8 * (p & 3));
     }
@@ -263,7 +322,12 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
   const int NOUT = 16 * NB;
   const int first = (2 * wave + (vl >> 3)) * kHE + (vl & 7);  // halo voxel of tap 0
   const int nz = min(kE, k.Ds - k.z0);
-  const bool rows = 2 * wave < k.Hs - k.y0;  // the wave has voxels
+  bool rows = 2 * wave < k.Hs - k.y0;  // the wave has voxels
+  unsigned planes = 0;                 // planes with voxels (packed)
+  if (kPack) {
+    planes = packed_positions(G.pz, k.rz, k.z0, G.D, G.dil);
+    rows = ((packed_positions(G.py, k.ry, k.y0, G.H, G.dil) >> (2 * wave)) & 3u) != 0;
+  }
   f32x4 acc[kE][NB];
 #pragma unroll
   for (int r = 0; r < kE; ++r)
@@ -292,7 +356,11 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
       for (int kw = 0; kw < 3; ++kw) {
 #pragma unroll
         for (int r = 0; r < kE; ++r) {
-          if (!decltype(whole)::value && r >= nz) break;
+          if (kPack) {
+            if (((planes >> r) & 1u) == 0) continue;
+          } else if (!decltype(whole)::value && r >= nz) {
+            break;
+          }
           const int v = at + kw + r * kHE * kHE;
           bf16x8 a;
           if (kFeat)
@@ -308,7 +376,7 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
     }
   };
   if (rows) {
-    if (nz == kE)
+    if (!kPack && nz == kE)
       products(std::true_type{});
     else
       products(std::false_type{});
@@ -336,7 +404,7 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
 #pragma unroll
     for (int i = 0; i < kOut; ++i) {
       const int p = (int)threadIdx.x + i * kConvThreads;
-      const long long g = inner_voxel(G, k, p >> 2);
+      const long long g = inner_voxel<kPack>(G, k, p >> 2);
       if (g < 0) continue;
       bf16x8 o = reinterpret_cast<const bf16x8 *>(lds)[p];
       if (mask) {
@@ -353,8 +421,8 @@ __global__ void __launch_bounds__(kConvThreads, 2) conv_block_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int vrow = 4 * kg + i;
-        const long long g = block_voxel(G, k, k.z0 + r, k.y0 + 2 * wave + (vrow >> 3),
-                                        k.x0 + (vrow & 7));
+        const long long g =
+            block_voxel<kPack>(G, k, r, 2 * wave + (vrow >> 3), vrow & 7);
         if (g >= 0) yf[g] = acc[r][0][i] + (bias ? bias[0] : 0.f);
       }
   }
@@ -407,6 +475,7 @@ constexpr int kTapsPerWave = 7;
 // block's loads are in flight under them.  2^20 voxels: 100 us (16 of them the
 // final adds; 76 with an eighth of the products), against 970 for one wave per
 // tap, channel block and 16 runs with 2-byte operand loads.
+template <bool kPack>
 __global__ void __launch_bounds__(kGThreads, 2) wgrad_block_kernel(
     BlockGeo G, const __bf16 *__restrict__ dy, const __bf16 *__restrict__ x,
     float *__restrict__ grad, size_t stride, size_t off_w, size_t off_b) {
@@ -416,18 +485,18 @@ __global__ void __launch_bounds__(kGThreads, 2) wgrad_block_kernel(
   constexpr int kXL = (4 * kGHalo + kGThreads - 1) / kGThreads, kDL = 4 * kGVox / kGThreads;
   bf16x8 px[kXL], pd[kDL];
   auto load = [&](int blk) {
-    const Block k = block_of<kGZ>(G, blk);
+    const Block k = block_of<kGZ, kPack>(G, blk);
 #pragma unroll
     for (int i = 0; i < kXL; ++i) {
       const int p = (int)threadIdx.x + i * kGThreads;
-      const long long g = p < 4 * kGHalo ? halo_voxel(G, k, p >> 2) : -1;
+      const long long g = p < 4 * kGHalo ? halo_voxel<kPack>(G, k, p >> 2) : -1;
       px[i] = bf16x8{};
       if (g >= 0) px[i] = *reinterpret_cast<const bf16x8 *>(x + g * kC + 8 * (p & 3));
     }
 #pragma unroll
     for (int i = 0; i < kDL; ++i) {
       const int p = (int)threadIdx.x + i * kGThreads;
-      const long long g = inner_voxel(G, k, p >> 2);
+      const long long g = inner_voxel<kPack>(G, k, p >> 2);
       pd[i] = bf16x8{};
       if (g >= 0) pd[i] = *reinterpret_cast<const bf16x8 *>(dy + g * kC + 8 * (p & 3));
     }
@@ -513,6 +582,7 @@ __global__ void __launch_bounds__(kGThreads, 2) wgrad_block_kernel(
 // The input is staged as planes shifted by each tap of the last axis, so that
 // an operand's 8 voxels are one aligned read.  Bound by reading dy once and
 // the final adds (42 us for 2^20 voxels; 59 with twice the workgroups).
+template <bool kPack>
 __global__ void __launch_bounds__(kGThreads) wgrad_first_kernel(
     BlockGeo G, const __bf16 *__restrict__ dy, const uint32_t *__restrict__ feat,
     float *__restrict__ grad, size_t stride, size_t off_w, size_t off_b) {
@@ -524,17 +594,17 @@ __global__ void __launch_bounds__(kGThreads) wgrad_first_kernel(
   uint32_t pf[kFL];
   bf16x8 pd[kDL];
   auto load = [&](int blk) {
-    const Block k = block_of<kGZ>(G, blk);
+    const Block k = block_of<kGZ, kPack>(G, blk);
 #pragma unroll
     for (int i = 0; i < kFL; ++i) {
       const int v = (int)threadIdx.x + i * kGThreads;
-      const long long g = v < kGHalo ? halo_voxel(G, k, v) : -1;
+      const long long g = v < kGHalo ? halo_voxel<kPack>(G, k, v) : -1;
       pf[i] = g >= 0 ? feat[g] : 0u;
     }
 #pragma unroll
     for (int i = 0; i < kDL; ++i) {
       const int p = (int)threadIdx.x + i * kGThreads;
-      const long long g = inner_voxel(G, k, p >> 2);
+      const long long g = inner_voxel<kPack>(G, k, p >> 2);
       pd[i] = bf16x8{};
       if (g >= 0) pd[i] = *reinterpret_cast<const bf16x8 *>(dy + g * kC + 8 * (p & 3));
     }
@@ -602,6 +672,7 @@ __global__ void __launch_bounds__(kGThreads) wgrad_first_kernel(
 // = sum_u dz[u - tap] x[u][ci], with the output gradient dz (one value per
 // voxel) staged in shifted planes.  Bound by reading x once (28 us for 2^20
 // voxels).  (The bias gradient, the sum of dz, comes with the loss.)
+template <bool kPack>
 __global__ void __launch_bounds__(kGThreads) wgrad_last_kernel(
     BlockGeo G, const uint16_t *__restrict__ dz, const __bf16 *__restrict__ x,
     float *__restrict__ grad, size_t stride, size_t off_w, int NOUT) {
@@ -613,17 +684,17 @@ __global__ void __launch_bounds__(kGThreads) wgrad_last_kernel(
   uint16_t pz[kFL];
   bf16x8 px[kDL];
   auto load = [&](int blk) {
-    const Block k = block_of<kGZ>(G, blk);
+    const Block k = block_of<kGZ, kPack>(G, blk);
 #pragma unroll
     for (int i = 0; i < kFL; ++i) {
       const int v = (int)threadIdx.x + i * kGThreads;
-      const long long g = v < kGHalo ? halo_voxel(G, k, v) : -1;
+      const long long g = v < kGHalo ? halo_voxel<kPack>(G, k, v) : -1;
       pz[i] = g >= 0 ? dz[g] : (uint16_t)0;
     }
 #pragma unroll
     for (int i = 0; i < kDL; ++i) {
       const int p = (int)threadIdx.x + i * kGThreads;
-      const long long g = inner_voxel(G, k, p >> 2);
+      const long long g = inner_voxel<kPack>(G, k, p >> 2);
       px[i] = bf16x8{};
       if (g >= 0) px[i] = *reinterpret_cast<const bf16x8 *>(x + g * kC + 8 * (p & 3));
     }
@@ -699,20 +770,21 @@ __global__ void __launch_bounds__(kGThreads) wgrad_last_kernel(
 // (27 of 32), one product per 16 voxels and 16 channels.  Bound by the mask
 // read and dx written once: 41 us for 2^20 voxels, 290 through 27 products
 // per 16 voxels of a 32-channel dz.
+template <bool kPack>
 __global__ void __launch_bounds__(kConvThreads) dgrad_last_kernel(
     BlockGeo G, const uint16_t *__restrict__ dz, const __bf16 *__restrict__ wb,
     const __bf16 *__restrict__ mask, __bf16 *__restrict__ dx) {
   constexpr int kHalo = kHE * kHE * kHE;
   __shared__ uint16_t zs[kHalo];
   __shared__ __align__(16) __bf16 out[kE * kE * kE * kC];
-  const Block k = block_of<kE>(G, blockIdx.x);
+  const Block k = block_of<kE, kPack>(G, blockIdx.x);
   if (k.z0 >= k.Ds || k.y0 >= k.Hs || k.x0 >= k.Ws) return;
   constexpr int kLoads = (kHalo + kConvThreads - 1) / kConvThreads;
   uint16_t vals[kLoads];
 #pragma unroll
   for (int i = 0; i < kLoads; ++i) {
     const int v = (int)threadIdx.x + i * kConvThreads;
-    const long long g = v < kHalo ? halo_voxel(G, k, v) : -1;
+    const long long g = v < kHalo ? halo_voxel<kPack>(G, k, v) : -1;
     vals[i] = g >= 0 ? dz[g] : (uint16_t)0;
   }
 #pragma unroll
@@ -762,7 +834,7 @@ __global__ void __launch_bounds__(kConvThreads) dgrad_last_kernel(
 #pragma unroll
   for (int i = 0; i < kE * kE * kE * 4 / kConvThreads; ++i) {
     const int p = (int)threadIdx.x + i * kConvThreads;
-    const long long g = inner_voxel(G, k, p >> 2);
+    const long long g = inner_voxel<kPack>(G, k, p >> 2);
     if (g < 0) continue;
     bf16x8 o = reinterpret_cast<const bf16x8 *>(out)[p];
     const bf16x8 m = *reinterpret_cast<const bf16x8 *>(mask + g * kC + 8 * (p & 3));
@@ -1176,23 +1248,53 @@ int pack(cmi_net *n) {
 }
 
 // Blocks of bz x 8 x 8 voxels over B samples of D x H x W at a dilation.
-BlockGeo block_geo(int B, int D, int H, int W, int dil, int bz) {
+//
+// Packed: where blocks of one sub-lattice each are more than the chip takes at a
+// time (two to a CU); fewer run side by side, and longer when packed.  Four
+// layers of one dilation, not packed and packed: 8 x 128 x 128, dilation 8, 2048
+// blocks 0.270 and 0.190 ms; 23 x 64 x 128, 8, 1024 blocks 0.232 and 0.224; 12 x
+// 64 x 64, 8, 512 blocks 0.115 and 0.140; 16 x 16 x 64, 8, 512 blocks 0.086 and
+// 0.120.
+//
+// Sparse: the 32-channel convolutions are faster voxel run by voxel run
+// (conv3_kernel) where the runs are about one to a SIMD (16 x 16 x 64, dilation 1,
+// 1024 runs: blocks 0.095, runs 0.088 ms; 12 x 12 x 128, 2, 1152 runs 0.100 and
+// 0.095; 9 x 31 x 96, 1, 1674 runs 0.101 and 0.105), and where voxels fill few of
+// the blocks' positions: packed 0.22 of them (64 x 64 x 96, dilation 24) 0.70 and
+// 0.60 ms, 0.30 (96^3, 36) 1.27 and 1.26, 0.39 (128^3, 43) 2.55 and 2.91; not
+// packed, which leaves empty planes out, 0.15 (128^3, 30) 3.40 and 2.99, 0.22
+// (96^3, 20) 1.24 and 1.31, 0.25 (64 x 64 x 128, 16) 0.66 and 0.79.
+BlockGeo block_geo(const cmi_net *n, int B, int D, int H, int W, int dil, int bz) {
   BlockGeo G;
   G.D = D;
   G.H = H;
   G.W = W;
   G.dil = dil;
-  G.nrz = std::min(dil, D);
-  G.nry = std::min(dil, H);
-  G.nrx = std::min(dil, W);
-  auto blocks = [&](int extent, int edge) {
+  // an axis: its residues (or groups of them), blocks and packing
+  auto axis = [&](int extent, int edge, bool pack, int &nr, int &nb, Residues &P) {
     const int sub = (extent + dil - 1) / dil;
-    return (sub + edge - 1) / edge;
+    P = Residues{std::min(dil, extent), 1, 0, 0};
+    // as many sub-lattices as fit with an empty position between neighbours
+    const int fit = std::min((edge + 1) / (sub + 1), P.res);
+    if (pack && fit > 1) {
+      P = Residues{P.res, fit, sub + 1, 256 / (sub + 1) + 1};
+      G.packed = true;
+    }
+    nr = (P.res + P.per_block - 1) / P.per_block;
+    nb = (sub + edge - 1) / edge;
   };
-  G.nbz = blocks(D, bz);
-  G.nby = blocks(H, kE);
-  G.nbx = blocks(W, kE);
-  G.nblocks = B * G.nrz * G.nry * G.nrx * G.nbz * G.nby * G.nbx;
+  auto blocks = [&](bool pack) {
+    G.packed = false;
+    axis(D, bz, pack, G.nrz, G.nbz, G.pz);
+    axis(H, kE, pack, G.nry, G.nby, G.py);
+    axis(W, kE, pack, G.nrx, G.nbx, G.px);
+    G.nblocks = B * G.nrz * G.nry * G.nrx * G.nbz * G.nby * G.nbx;
+  };
+  blocks(false);
+  if (G.nblocks > 2 * n->num_cus) blocks(true);
+  const double voxels = (double)B * D * H * W;
+  G.sparse = voxels <= 16. * 5. * n->num_cus ||
+             voxels < (G.packed ? 0.3 : 0.2) * G.nblocks * bz * kE * kE;
   return G;
 }
 
@@ -1221,35 +1323,31 @@ int forward(cmi_net *n, int B, int D, int H, int W, float *zout) {
   if ((size_t)B * D * H * W == 0) return CMI_OK;  // nothing to compute, no empty grids
   const int nrun = B * D * H * (W / 16);
   const unsigned runs = grid_for((size_t)nrun, 4, 1u << 30);  // one wave per run
-  const __bf16 *const in = reinterpret_cast<const __bf16 *>(n->in);
   for (int l = 0; l < kLayers; ++l) {
     const float *bias = n->p + n->off_b[l];
-    const int dil = n->dil[l];
-    if (n->tiled) {
-      const BlockGeo G = block_geo(B, D, H, W, dil, kE);
-#define CMI_CONV(NB, FEAT, X, Y, YF, RELU)                                                \
-  hipLaunchKernelGGL((conv_block_kernel<NB, FEAT>), dim3(G.nblocks), dim3(kConvThreads), 0, \
-                     n->stream, G, X, n->wf[l], bias, Y, YF, (const __bf16 *)nullptr, RELU)
+    const int dil = n->dil[l], relu = l < kLayers - 1;
+    const __bf16 *const x = l == 0 ? reinterpret_cast<const __bf16 *>(n->in) : n->act[l];
+    __bf16 *const y = relu ? n->act[l + 1] : nullptr;
+    float *const yf = relu ? nullptr : zout;
+    const BlockGeo G = block_geo(n, B, D, H, W, dil, kE);
+    if (n->tiled && !G.sparse) {
+      const bool pk = G.packed;
+      auto *conv = pk ? conv_block_kernel<2, false, true> : conv_block_kernel<2, false, false>;
       if (l == 0)
-        CMI_CONV(2, true, in, n->act[1], (float *)nullptr, 1);
-      else if (l < kLayers - 1)
-        CMI_CONV(2, false, n->act[l], n->act[l + 1], (float *)nullptr, 1);
-      else
-        CMI_CONV(1, false, n->act[l], (__bf16 *)nullptr, zout, 0);
-#undef CMI_CONV
+        conv = pk ? conv_block_kernel<2, true, true> : conv_block_kernel<2, true, false>;
+      else if (l == kLayers - 1)
+        conv = pk ? conv_block_kernel<1, false, true> : conv_block_kernel<1, false, false>;
+      hipLaunchKernelGGL(conv, dim3(G.nblocks), dim3(kConvThreads), 0, n->stream, G, x,
+                         n->wf[l], bias, y, yf, (const __bf16 *)nullptr, relu);
       continue;
     }
+    auto *run = conv3_kernel<2, false>;
     if (l == 0)
-      hipLaunchKernelGGL((conv3_kernel<2, true>), dim3(runs), dim3(256), 0, n->stream, in,
-                         n->wf[l], bias, nrun, D, H, W, dil, n->act[1], (float *)nullptr, 1);
-    else if (l < kLayers - 1)
-      hipLaunchKernelGGL((conv3_kernel<2, false>), dim3(runs), dim3(256), 0, n->stream,
-                         n->act[l], n->wf[l], bias, nrun, D, H, W, dil, n->act[l + 1],
-                         (float *)nullptr, 1);
-    else
-      hipLaunchKernelGGL((conv3_kernel<1, false>), dim3(runs), dim3(256), 0, n->stream,
-                         n->act[l], n->wf[l], bias, nrun, D, H, W, dil, (__bf16 *)nullptr, zout,
-                         0);
+      run = conv3_kernel<2, true>;
+    else if (l == kLayers - 1)
+      run = conv3_kernel<1, false>;
+    hipLaunchKernelGGL(run, dim3(runs), dim3(256), 0, n->stream, x, n->wf[l], bias, nrun, D, H,
+                       W, dil, y, yf, (const __bf16 *)nullptr, relu);
   }
   NET_TRY(n, hipGetLastError());
   return CMI_OK;
@@ -1274,33 +1372,46 @@ int backward(cmi_net *n, int B, int D, int H, int W) {
   const size_t nvox = (size_t)B * D * H * W;
   const uint16_t *const dz = reinterpret_cast<const uint16_t *>(n->dz);
   const int last = kLayers - 1;
+  const int nrun = B * D * H * (W / 16);
+  const unsigned runs = grid_for((size_t)nrun, 4, 1u << 30);  // one wave per run
   hipLaunchKernelGGL(mse_kernel, dim3(grid_for(nvox, 1024, 512)), dim3(256), 0, n->stream,
                      n->z, n->tgt, nvox, n->w_pos, n->dz, n->g, n->grad_stride, n->nparam,
                      n->off_b[last]);
   __bf16 *dy = n->dact[0], *dx = n->dact[1];
   // without voxels the mean loss is NaN and the gradients stay 0
   for (int l = nvox ? last : -1; l >= 0; --l) {
-    const BlockGeo Gw = block_geo(B, D, H, W, n->dil[l], kGZ);
-    const BlockGeo Gx = block_geo(B, D, H, W, n->dil[l], kE);
+    const BlockGeo Gw = block_geo(n, B, D, H, W, n->dil[l], kGZ);
+    const BlockGeo Gx = block_geo(n, B, D, H, W, n->dil[l], kE);
     const unsigned wg = grad_grid(n, Gw);
     if (l == last) {
-      hipLaunchKernelGGL(wgrad_last_kernel, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dz,
-                         n->act[l], n->g, n->grad_stride, n->off_w[l], nout_of(l));
-      hipLaunchKernelGGL(dgrad_last_kernel, dim3(Gx.nblocks), dim3(kConvThreads), 0, n->stream,
-                         Gx, dz, n->wb[l], n->act[l], dy);
+      auto *wgrad = Gw.packed ? wgrad_last_kernel<true> : wgrad_last_kernel<false>;
+      hipLaunchKernelGGL(wgrad, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dz, n->act[l],
+                         n->g, n->grad_stride, n->off_w[l], nout_of(l));
+      auto *dgrad = Gx.packed ? dgrad_last_kernel<true> : dgrad_last_kernel<false>;
+      hipLaunchKernelGGL(dgrad, dim3(Gx.nblocks), dim3(kConvThreads), 0, n->stream, Gx, dz,
+                         n->wb[l], n->act[l], dy);
       continue;
     }
     if (l == 0) {
-      hipLaunchKernelGGL(wgrad_first_kernel, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dy,
-                         n->in, n->g, n->grad_stride, n->off_w[l], n->off_b[l]);
+      auto *wgrad = Gw.packed ? wgrad_first_kernel<true> : wgrad_first_kernel<false>;
+      hipLaunchKernelGGL(wgrad, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dy, n->in, n->g,
+                         n->grad_stride, n->off_w[l], n->off_b[l]);
       continue;
     }
-    hipLaunchKernelGGL(wgrad_block_kernel, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dy,
-                       n->act[l], n->g, n->grad_stride, n->off_w[l], n->off_b[l]);
+    auto *wgrad = Gw.packed ? wgrad_block_kernel<true> : wgrad_block_kernel<false>;
+    hipLaunchKernelGGL(wgrad, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dy, n->act[l], n->g,
+                       n->grad_stride, n->off_w[l], n->off_b[l]);
     // dx = conv(dy, flipped transposed W), masked by the ReLU of layer l-1
-    hipLaunchKernelGGL((conv_block_kernel<2, false>), dim3(Gx.nblocks), dim3(kConvThreads), 0,
-                       n->stream, Gx, dy, n->wb[l], (const float *)nullptr, dx, (float *)nullptr,
-                       n->act[l], 0);
+    if (Gx.sparse) {
+      hipLaunchKernelGGL((conv3_kernel<2, false>), dim3(runs), dim3(256), 0, n->stream, dy,
+                         n->wb[l], (const float *)nullptr, nrun, D, H, W, n->dil[l], dx,
+                         (float *)nullptr, n->act[l], 0);
+    } else {
+      auto *conv =
+          Gx.packed ? conv_block_kernel<2, false, true> : conv_block_kernel<2, false, false>;
+      hipLaunchKernelGGL(conv, dim3(Gx.nblocks), dim3(kConvThreads), 0, n->stream, Gx, dy,
+                         n->wb[l], (const float *)nullptr, dx, (float *)nullptr, n->act[l], 0);
+    }
     std::swap(dy, dx);
   }
   NET_TRY(n, hipGetLastError());
