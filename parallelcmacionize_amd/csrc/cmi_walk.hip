@@ -17,6 +17,8 @@
 //             J accumulates the path length in units of Delta_0 (FP64).
 #include <float.h>
 
+#include <algorithm>
+
 #include "cmi_device.hpp"
 #include "cmi_internal.hpp"
 
@@ -482,22 +484,20 @@ __global__ void walk_list_kernel(GridDev g, Mode m, PhotonRec *p,
 //          the hop into the neighbour subgrid, the reemission, the end of the
 //          packet, and the next packet (a wave-aggregated ticket, then the
 //          emission);
-//   walk   crossings only, until kServeBatch of the walking lanes have left
-//          their subgrid or ended (or none walks).
+//   walk   crossings only, until as many of the walking lanes as half of those
+//          that take packets have left their subgrid or ended (or none walks).
 // The serve phase is expensive (an emission is about 1000 instructions with
 // its FP64 sincos and logarithm, a hop reads the neighbour table and then two
 // anchors), and some lane of 64 needs it after nearly every crossing.  Served
-// 8 at a time instead of 32 the three transports above take 9.3 ms instead of
+// 8 at a time instead of 32 (of 64) the three transports above take 9.3 ms instead of
 // 7.4; 48 and 64 at a time take the same.  Four workgroups a CU (128 VGPRs;
 // 141 without the bound) is what the LDS table allows: 5 % less time.
 // ---------------------------------------------------------------------------
-constexpr int kServeBatch = 32;
-
 template <class Mode>
 __global__ void __launch_bounds__(256, 4) walk_emit_kernel(
     GridDev g, Mode m, const SourcesDev *__restrict__ S, uint64_t npackets,
     uint32_t iteration, uint32_t key0, uint32_t key1, double sigma,
-    int max_steps, int max_hops, ReemitDraws re, Counters *cnt) {
+    int max_steps, int max_hops, ReemitDraws re, Counters *cnt, int lanes) {
   using T = typename Mode::real;
   __shared__ HotTable hot;
   for (int i = threadIdx.x; i < (int)kHotCrossings * kHotPart; i += blockDim.x) {
@@ -510,7 +510,8 @@ __global__ void __launch_bounds__(256, 4) walk_emit_kernel(
   Walker<T> w;
   bool live = false;       // walking
   bool owned = false;      // the lane holds a packet
-  bool exhausted = false;  // no packet is left for the lane
+  bool exhausted = lane >= lanes;  // no packet is left for the lane
+  const int serve_batch = (lanes + 1) >> 1;
   int r = kContinue;       // how the last walk ended
   int steps = 0;           // crossings of this subgrid visit
   int leg_hops = 0;        // subgrid visits since the emission or reemission
@@ -586,7 +587,7 @@ __global__ void __launch_bounds__(256, 4) walk_emit_kernel(
     if (!__any(owned)) break;
     // ---- walk ----
     int nlive = __popcll(__ballot(live));
-    const int stop_at = max(nlive - kServeBatch, 0);
+    const int stop_at = max(nlive - serve_batch, 0);
     while (nlive > stop_at) {
       if (live) {
         if (steps < max_steps) {
@@ -686,14 +687,25 @@ hipError_t launch_walk_emit(const GridDev &g, const FieldsDev &f, int prec,
   const int max_steps = g.sc[0] + g.sc[1] + g.sc[2] + 8;
   const int max_hops = 4 * (g.nsub[0] + g.nsub[1] + g.nsub[2]) + 16;
   const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+  // Few packets: as many lanes of a wave take packets as give work to one wave
+  // per SIMD (an eighth of the default grid's), and no more waves are launched
+  // than that takes.  A wave of 64 serves its lanes by halves, so each waits for
+  // others, and every idle wave still asks the one ticket counter (8192 of them
+  // take 90 us).  64^3 cells, 1 packet 0.138 -> 0.046 ms, 1e4 0.205 -> 0.128, 1e5
+  // 0.300 -> 0.220; 128^3, 1000 packets 0.525 -> 0.245; from 3e5 on the same.  With
+  // one lane in each of all 8192 waves 1e4 packets take 0.27 ms.
+  const uint64_t few = std::max(1, blocks / 2);
+  const int lanes = (int)std::min<uint64_t>(64, (npackets + few - 1) / few);
+  const uint64_t waves = lanes ? (npackets + lanes - 1) / lanes : 1;
+  blocks = (int)std::min<uint64_t>(blocks, (waves + 3) / 4);
   if (prec == 0) {
     hipLaunchKernelGGL(walk_emit_kernel<Mode64>, dim3(blocks), dim3(256), 0,
                        st, g, Mode64{f.n, f.xn, f.J}, S, npackets, iteration,
-                       k0, k1, sigma, max_steps, max_hops, re, cnt);
+                       k0, k1, sigma, max_steps, max_hops, re, cnt, lanes);
   } else {
     hipLaunchKernelGGL(walk_emit_kernel<Mode32>, dim3(blocks), dim3(256), 0,
                        st, g, Mode32{f.kappa, f.J}, S, npackets, iteration,
-                       k0, k1, sigma, max_steps, max_hops, re, cnt);
+                       k0, k1, sigma, max_steps, max_hops, re, cnt, lanes);
   }
   return hipGetLastError();
 }
