@@ -394,13 +394,12 @@ int cmi_set_fields(cmi_ctx *c, const double *nH, const double *xn) {
   // on the context's stream, behind what is queued there: a restriction or
   // prolongation into this context, or out of it (which makes this stream wait
   // until the other context's has read the fields)
-  CMI_TRY_HIP(c, put_fields(c, CellField{const_cast<double *>(nH), c->f.n, 1.},
-                            CellField{const_cast<double *>(xn), c->f.xn, 1.}));
-  if (c->precision == CMI_PREC_FP32) {
-    CMI_TRY_HIP(c, launch_kappa(c->f, c->ncell_total, c->sigma * delta0(c),
-                                c->stream));
-  }
+  hipError_t upload = put_fields(c, CellField{const_cast<double *>(nH), c->f.n, 1.},
+                                 CellField{const_cast<double *>(xn), c->f.xn, 1.});
+  if (upload == hipSuccess && c->precision == CMI_PREC_FP32)
+    upload = launch_kappa(c->f, c->ncell_total, c->sigma * delta0(c), c->stream);
   CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
+  CMI_TRY_HIP(c, upload);
   return CMI_OK;
 }
 
@@ -408,8 +407,10 @@ int cmi_set_intensity(cmi_ctx *c, const double *J) {
   if (!c || !J) return CMI_ERR_ARG;
   (void)hipSetDevice(c->device);
   const double scale = c->precision == CMI_PREC_FP32 ? 1. / (c->sigma * delta0(c)) : 1.;
-  CMI_TRY_HIP(c, put_fields(c, CellField{const_cast<double *>(J), c->f.J, scale}));
+  const hipError_t upload =
+      put_fields(c, CellField{const_cast<double *>(J), c->f.J, scale});
   CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
+  CMI_TRY_HIP(c, upload);
   return CMI_OK;
 }
 

@@ -46,7 +46,9 @@ class Stage {
  public:
   ~Stage();
   // Fields of n cells between the caller's order and the device's, behind
-  // what is queued on the stream; complete on return.
+  // what is queued on the stream.  A download is complete on return.  After an
+  // upload the caller's arrays are free; it waits for the stream before the
+  // next transfer.
   hipError_t upload_cells(int device, hipStream_t st, const CellOrder &o, size_t n,
                           const CellField *fields, int nfields);
   hipError_t download_cells(int device, hipStream_t st, const CellOrder &o, size_t n,
@@ -56,12 +58,14 @@ class Stage {
   static constexpr int kThreads = 4;            // host threads of a large transfer
   static constexpr int kSlots = 2 * kThreads;   // two per thread
   static constexpr size_t kPiece = 1u << 20;    // bytes of a slot
+  static constexpr size_t kSmall = 1u << 17;    // bytes of a small download
   unsigned char *h_[kSlots] = {};
   hipEvent_t ev_[kSlots] = {};
 
   hipError_t ensure(int slots);
   template <class Piece>
-  hipError_t run(int device, size_t bytes, int arrays, const Piece &piece);
+  hipError_t run(int device, hipStream_t st, bool upload, size_t bytes, int arrays,
+                 const Piece &piece);
 };
 
 }  // namespace cmi
