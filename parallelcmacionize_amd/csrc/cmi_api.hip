@@ -352,6 +352,7 @@ void cmi_destroy(cmi_ctx *c) {
   hipFree(c->d_partial);
   if (c->ev0) hipEventDestroy(c->ev0);
   if (c->ev1) hipEventDestroy(c->ev1);
+  if (c->ev_read) hipEventDestroy(c->ev_read);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
 }

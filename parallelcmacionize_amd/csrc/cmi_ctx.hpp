@@ -42,6 +42,7 @@ struct cmi_ctx {
   uint64_t reemit_seed = 0;       // key of the list transports' reemission draws
   uint32_t reemit_iteration = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  hipEvent_t ev_read = nullptr;  // what this context queued has read another's fields
   double kernel_time_sum = 0.;
   uint64_t kernel_calls = 0;
   int kernel_timing = 1;  // record the tiles engine's per-round process events

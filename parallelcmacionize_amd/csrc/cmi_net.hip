@@ -1822,14 +1822,12 @@ static int coarse_factor(const cmi_ctx *fine, const cmi_ctx *coarse) {
 
 // What is queued on `reader`'s stream reads `source`'s fields: work that
 // `source` gets from here on waits for it.
-static hipError_t hold_fields(cmi_ctx *source, const cmi_ctx *reader) {
-  hipEvent_t read = nullptr;
-  hipError_t e = hipEventCreateWithFlags(&read, hipEventDisableTiming);
-  if (e != hipSuccess) return e;
-  e = hipEventRecord(read, reader->stream);
-  if (e == hipSuccess) e = hipStreamWaitEvent(source->stream, read, 0);
-  const hipError_t d = hipEventDestroy(read);  // released once it has passed
-  return e == hipSuccess ? d : e;
+static hipError_t hold_fields(cmi_ctx *source, cmi_ctx *reader) {
+  hipError_t e = hipSuccess;
+  if (!reader->ev_read) e = hipEventCreateWithFlags(&reader->ev_read, hipEventDisableTiming);
+  if (e == hipSuccess) e = hipEventRecord(reader->ev_read, reader->stream);
+  if (e == hipSuccess) e = hipStreamWaitEvent(source->stream, reader->ev_read, 0);
+  return e;
 }
 
 int cmi_restrict_density(cmi_ctx *fine, cmi_ctx *coarse) {
