@@ -171,7 +171,10 @@ struct BlockGeo {
   int nbz, nby, nbx;  // blocks per axis of the largest sub-lattice
   int nblocks;
   bool packed;        // some axis has several residues to a block
-  bool sparse;        // convolutions run by run instead (block_geo)
+  // for the choice between blocks and runs (block_geo)
+  bool sparse;    // few of the blocks' positions hold voxels
+  bool few_runs;  // about a run per SIMD
+  bool one_wave;  // all blocks at a time
   Residues pz, py, px;
 };
 
@@ -1256,14 +1259,18 @@ int pack(cmi_net *n) {
 // 64 x 64, 8, 512 blocks 0.115 and 0.140; 16 x 16 x 64, 8, 512 blocks 0.086 and
 // 0.120.
 //
-// Sparse: the 32-channel convolutions are faster voxel run by voxel run
-// (conv3_kernel) where the runs are about one to a SIMD (16 x 16 x 64, dilation 1,
-// 1024 runs: blocks 0.095, runs 0.088 ms; 12 x 12 x 128, 2, 1152 runs 0.100 and
-// 0.095; 9 x 31 x 96, 1, 1674 runs 0.101 and 0.105), and where voxels fill few of
-// the blocks' positions: packed 0.22 of them (64 x 64 x 96, dilation 24) 0.70 and
+// Runs instead of blocks (by_runs): an inference is faster voxel run by voxel run
+// (conv3_kernel, a tenth of the code) where the runs are about one to a SIMD (16 x
+// 16 x 64, dilation 1, 1024 runs: blocks 0.095, runs 0.088 ms; 12 x 12 x 128, 2,
+// 1152 runs 0.100 and 0.095; 9 x 31 x 96, 1, 1674 runs 0.101 and 0.105), and where
+// voxels fill few of the blocks' positions: packed 0.22 of them (64 x 64 x 96, dilation 24) 0.70 and
 // 0.60 ms, 0.30 (96^3, 36) 1.27 and 1.26, 0.39 (128^3, 43) 2.55 and 2.91; not
 // packed, which leaves empty planes out, 0.15 (128^3, 30) 3.40 and 2.99, 0.22
-// (96^3, 20) 1.24 and 1.31, 0.25 (64 x 64 x 128, 16) 0.66 and 0.79.
+// (96^3, 20) 1.24 and 1.31, 0.25 (64 x 64 x 128, 16) 0.66 and 0.79.  In training,
+// where one step follows the other, runs are faster only where the blocks are
+// also more than the chip takes at a time (8 steps on a crop of 8 x 8 x 32: blocks
+// 1.11, runs forward and back 1.19 ms; 4 steps on two of 64^3 at dilations of 16,
+// 4096 blocks: 5.97 and 4.77).
 BlockGeo block_geo(const cmi_net *n, int B, int D, int H, int W, int dil, int bz) {
   BlockGeo G;
   G.D = D;
@@ -1293,9 +1300,15 @@ BlockGeo block_geo(const cmi_net *n, int B, int D, int H, int W, int dil, int bz
   blocks(false);
   if (G.nblocks > 2 * n->num_cus) blocks(true);
   const double voxels = (double)B * D * H * W;
-  G.sparse = voxels <= 16. * 5. * n->num_cus ||
-             voxels < (G.packed ? 0.3 : 0.2) * G.nblocks * bz * kE * kE;
+  G.sparse = voxels < (G.packed ? 0.3 : 0.2) * G.nblocks * bz * kE * kE;
+  G.few_runs = voxels <= 16. * 5. * n->num_cus;
+  G.one_wave = G.nblocks <= 2 * n->num_cus;
   return G;
+}
+
+// Whether a 32-channel convolution goes run by run (block_geo).
+bool by_runs(const BlockGeo &G, bool training) {
+  return training ? G.sparse && !G.one_wave : G.sparse || G.few_runs;
 }
 
 unsigned grid_for(size_t items, unsigned per_block, unsigned cap = 65535) {
@@ -1318,8 +1331,9 @@ void input_features(cmi_net *n, const float *feat, int B, const int dim[3]) {
   }
 }
 
-// forward over n->in (B samples of D x H x W) -> zout
-int forward(cmi_net *n, int B, int D, int H, int W, float *zout) {
+// forward over n->in (B samples of D x H x W) -> zout; training: a backward
+// pass follows
+int forward(cmi_net *n, int B, int D, int H, int W, float *zout, bool training) {
   if ((size_t)B * D * H * W == 0) return CMI_OK;  // nothing to compute, no empty grids
   const int nrun = B * D * H * (W / 16);
   const unsigned runs = grid_for((size_t)nrun, 4, 1u << 30);  // one wave per run
@@ -1330,7 +1344,7 @@ int forward(cmi_net *n, int B, int D, int H, int W, float *zout) {
     __bf16 *const y = relu ? n->act[l + 1] : nullptr;
     float *const yf = relu ? nullptr : zout;
     const BlockGeo G = block_geo(n, B, D, H, W, dil, kE);
-    if (n->tiled && !G.sparse) {
+    if (n->tiled && !by_runs(G, training)) {
       const bool pk = G.packed;
       auto *conv = pk ? conv_block_kernel<2, false, true> : conv_block_kernel<2, false, false>;
       if (l == 0)
@@ -1402,7 +1416,7 @@ int backward(cmi_net *n, int B, int D, int H, int W) {
     hipLaunchKernelGGL(wgrad, dim3(wg), dim3(kGThreads), 0, n->stream, Gw, dy, n->act[l], n->g,
                        n->grad_stride, n->off_w[l], n->off_b[l]);
     // dx = conv(dy, flipped transposed W), masked by the ReLU of layer l-1
-    if (Gx.sparse) {
+    if (by_runs(Gx, true)) {
       hipLaunchKernelGGL((conv3_kernel<2, false>), dim3(runs), dim3(256), 0, n->stream, dy,
                          n->wb[l], (const float *)nullptr, nrun, D, H, W, n->dil[l], dx,
                          (float *)nullptr, n->act[l], 0);
@@ -1669,7 +1683,7 @@ int cmi_net_train(cmi_net *n, int steps, int batch, const int crop[3], float lr,
                          n->tgt + (size_t)b0 * cv);
     }
     zero_grad(n);
-    rc = forward(n, batch, crop[0], crop[1], crop[2], n->z);
+    rc = forward(n, batch, crop[0], crop[1], crop[2], n->z, true);
     if (rc != CMI_OK) return rc;
     rc = backward(n, batch, crop[0], crop[1], crop[2]);
     if (rc != CMI_OK) return rc;
@@ -1713,7 +1727,7 @@ int cmi_net_loss_and_grad(cmi_net *n, const float *feat, const float *target, in
   }
   input_features(n, df, B, dim);
   zero_grad(n);
-  rc = forward(n, B, dim[0], dim[1], dim[2], n->z);
+  rc = forward(n, B, dim[0], dim[1], dim[2], n->z, true);
   if (rc == CMI_OK) rc = backward(n, B, dim[0], dim[1], dim[2]);
   if (rc == CMI_OK) {
     hipLaunchKernelGGL(sum_grad_kernel, dim3(grid_for(n->nparam, 256, 1024)), dim3(256), 0,
@@ -1749,7 +1763,7 @@ int cmi_net_predict(cmi_net *n, const float *feat, const int dim[3], float *logi
   }
   NET_TRY(n, hipMemcpy(n->feat_tmp, feat, nv * 2 * sizeof(float), hipMemcpyHostToDevice));
   input_features(n, n->feat_tmp, 1, dim);
-  rc = forward(n, 1, dim[0], dim[1], dim[2], n->z);
+  rc = forward(n, 1, dim[0], dim[1], dim[2], n->z, false);
   if (rc != CMI_OK) return rc;
   NET_TRY(n, hipMemcpyAsync(logits, n->z, nv * sizeof(float), hipMemcpyDeviceToHost, n->stream));
   NET_TRY(n, hipStreamSynchronize(n->stream));
@@ -1793,7 +1807,7 @@ int cmi_net_warm_start(cmi_net *n, cmi_ctx *c, double luminosity, uint64_t npack
                      (const double *)c->f.xn, n->mode, D, H, W,
                      context_jconv(c, luminosity, npackets), n->mean[0], n->scale[0],
                      n->mean[1], n->scale[1], n->in, (float *)nullptr);
-  rc = forward(n, 1, D, H, W, n->z);
+  rc = forward(n, 1, D, H, W, n->z, false);
   if (rc != CMI_OK) return rc;
   const bool fp32 = c->precision == CMI_PREC_FP32;
   hipLaunchKernelGGL(ctx_apply_kernel, dim3(grid_for(nv, 256, 8192)), dim3(256), 0, n->stream,
