@@ -93,9 +93,10 @@ typedef struct {
                         them out and reloads together (1..64) */
   int chunk_min;     /* tiles: packets of one tile one workgroup visit
                         takes (a tile's packets are split in such chunks;
-                        >= 256, default 8192); a round with fewer packets
-                        than a quarter of the resident workgroups' worth of
-                        such chunks uses smaller ones (down to 256) */
+                        default 8192, values below 256 and above 2^26 count
+                        as those); a round with fewer packets than such a
+                        chunk for every resident workgroup uses smaller ones
+                        (down to 256) */
   int walk_blocks;   /* walk: persistent grid size */
   int lds_fp32;      /* tiles: 1 = FP32 LDS accumulators for J (flushed into
                         FP64; slower on gfx950), 0 = 64-bit fixed point */

@@ -1085,15 +1085,16 @@ __global__ void __launch_bounds__(kThreads, kTile ? 6 : 1) tiles_process_kernel(
   __shared__ uint32_t s_face[7];  // the visit's exits through each face, and in all
 
   const int lane = threadIdx.x & 63;
-  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const uint32_t ndesc = round->visits;
   if (blockIdx.x >= ndesc) return;  // no visit for this workgroup
   const int T0 = kTile ? kTile : G.T[0], T1 = kTile ? kTile : G.T[1],
             T2 = kTile ? kTile : G.T[2];
   const int st0 = (T1 * T2) << 2, st1 = T2 << 2;  // byte strides
   // counts of this launch: the wave's in scalar registers (from the lane
-  // masks), crossings, errors and reemissions per lane (32 bits: a lane walks
-  // at most a few hundred thousand crossings per launch)
+  // masks), crossings, errors and reemissions per lane.  32 bits: a straight
+  // flight crosses at most 128 cells of a tile, so a lane's share of 2^32 packets
+  // in one tile is below 2^26 crossings; a lane that reemission keeps in its tile
+  // for 2^32 would walk for minutes.
   uint32_t w_hops = 0, w_abs = 0, w_esc = 0;
   uint32_t my_cross = 0, my_err = 0, my_re = 0;
 
@@ -1702,11 +1703,10 @@ struct TilesEngine {
   int turn = 0;
   Desc *desc = nullptr;        // work descriptors of the round
   Round *round = nullptr;
-  // [3]: packets of the round being planned, packets of the round just
-  // processed, number of plans that found packets
+  // [2]: packets of the round being planned, number of plans that found packets
   uint32_t *total = nullptr;
   unsigned *ticket = nullptr;
-  uint32_t *h_total = nullptr;  // pinned, [3]
+  uint32_t *h_total = nullptr;  // pinned, [2]
   SrcTile *src_tile = nullptr;  // each source's start tile, cell and round-0 offset
   int tile_key[3] = {0, 0, 0};
   std::vector<hipEvent_t> ev;   // start/stop of every process launch
@@ -1789,9 +1789,6 @@ static std::vector<ProbGeo> ctx_problems(const cmi_ctx *c) {
 constexpr int kReemitRoundCap = 100000;
 constexpr size_t kLdsBytes = 160 * 1024;  // LDS of one CU on gfx950
 
-// The walk-state layout of a tile shape (WalkLayout); bits() of the result
-// is at most 32 for every tile set_tile accepts.
-
 static TileGeo make_geo(const cmi_ctx *c, const TilesEngine *e) {
   TileGeo G{};
   for (int a = 0; a < 3; ++a) {
@@ -1869,9 +1866,9 @@ static int ensure_engine(cmi_ctx *c, const std::vector<ProbGeo> &probs,
   if (err == hipSuccess) err = hipMalloc(&e->cursor, ntiles * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->desc, e->desc_cap * sizeof(Desc));
   if (err == hipSuccess) err = hipMalloc(&e->round, 2 * sizeof(Round));
-  if (err == hipSuccess) err = hipMalloc(&e->total, 3 * sizeof(uint32_t));
+  if (err == hipSuccess) err = hipMalloc(&e->total, 2 * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->ticket, sizeof(unsigned));
-  if (err == hipSuccess) err = hipHostMalloc(&e->h_total, 3 * sizeof(uint32_t));
+  if (err == hipSuccess) err = hipHostMalloc(&e->h_total, 2 * sizeof(uint32_t));
   if (err == hipSuccess) err = hipMalloc(&e->src_tile, kMaxSetSources * sizeof(SrcTile));
   if (err == hipSuccess) err = hipMalloc(&e->d_probs, np * sizeof(ProbGeo));
   if (err == hipSuccess) err = hipMalloc(&e->d_tile_prob, ntiles * sizeof(uint16_t));
@@ -2029,7 +2026,7 @@ static void launch_walkout(cmi_ctx *c, const TileGeo &G, const RoundCfg &R,
 }
 
 // Arguments of the next plan, which takes the turn.  nonempty: count the plans
-// that find packets (total[2]) -- the rounds after round 0 that had work.
+// that find packets (total[1]) -- the rounds after round 0 that had work.
 static PlanArgs next_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool track,
                           bool nonempty) {
   TilesEngine *e = c->tiles;
@@ -2051,7 +2048,7 @@ static PlanArgs next_plan(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool 
   A.prob_round = track ? e->d_prob_round : nullptr;
   A.prob_time = e->d_prob_time;
   A.round_ctr = e->d_round_ctr;
-  A.nonempty = nonempty ? e->total + 2 : nullptr;
+  A.nonempty = nonempty ? e->total + 1 : nullptr;
   return A;
 }
 
@@ -2115,19 +2112,19 @@ static int run_rounds(cmi_ctx *c, const TileGeo &G, const RoundCfg &R, bool with
       std::swap(e->P[0], e->P[1]);
       if (with_pid) std::swap(e->pid[0], e->pid[1]);
     }
-    CMI_TRY_HIP(c, hipMemcpyAsync(e->h_total, e->total, 3 * sizeof(uint32_t),
+    CMI_TRY_HIP(c, hipMemcpyAsync(e->h_total, e->total, 2 * sizeof(uint32_t),
                                   hipMemcpyDeviceToHost, c->stream));
     CMI_TRY_HIP(c, hipStreamSynchronize(c->stream));
     drained = e->h_total[0] == 0;
     if (!drained && e->h_total[0] <= R.finish_max) {
       // few packets left: one launch walks them to the end (the plan that
-      // found them counted this round in total[2])
+      // found them counted this round in total[1])
       launch_walkout(c, G, R, with_pid, po);
       CMI_TRY_HIP(c, hipGetLastError());
       drained = true;
     }
   }
-  if (rounds_out) *rounds_out = r == 0 ? 1u : 1u + e->h_total[2];
+  if (rounds_out) *rounds_out = r == 0 ? 1u : 1u + e->h_total[1];
   if (!drained) return fail(c, CMI_ERR_DIRECTION, "tiles engine: round limit reached");
   // device time of every process launch (the dominant kernel; walk-out
   // launches are not among them)
@@ -2201,7 +2198,7 @@ int tiles_transport(cmi_ctx *c, uint64_t npackets, uint64_t seed,
   // emission fills the records and the index list
   e->turn = 0;
   hipLaunchKernelGGL(tiles_source_hist_kernel, dim3(1), dim3(256), 0, c->stream, G,
-                     e->d_src, e->hist, e->total + 2, e->src_tile);
+                     e->d_src, e->hist, e->total + 1, e->src_tile);
   launch_first_plan(c, G, R, false);
   const unsigned eb = (unsigned)((npackets + 255) / 256);
   hipLaunchKernelGGL(tiles_emit_kernel, dim3(eb), dim3(256), 0, c->stream, G, e->d_src,
@@ -2275,7 +2272,7 @@ int tiles_transport_packets(cmi_ctx *c, cmi_photon *p, const uint32_t *start_sub
   e->turn = 0;
   hipLaunchKernelGGL(zero_u32_kernel, dim3(64), dim3(256), 0, c->stream, e->hist,
                      (size_t)G.ntiles);
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, c->stream, e->total + 2,
+  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, c->stream, e->total + 1,
                      (size_t)1);
   hipLaunchKernelGGL(tiles_load_list_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256),
                      0, c->stream, G, c->g, dp, ds, n, e->P[0], e->dest, e->pid[0],
